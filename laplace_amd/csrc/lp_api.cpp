@@ -171,20 +171,29 @@ static int check_shape(uint32_t type, const void* w, int M, int K, int N) {
     return LP_OK;
 }
 
-// Whether M > 16 rows run on the tiled GEMM. Q4_K at small prefill sizes
-// runs faster as 16-row chunks on the int8 MFMA kernel (one weight pass per
-// chunk) than on the GEMM's 64-token tiles (measured per call at
-// N x K = 14336 x 4096 / 4096 x 14336: M=17 32 vs 49 and 52 vs 136 us;
-// M=32 49 vs 54 and 82 vs 142; M=48 71 vs 59 and 122 vs 149; M=64 94 vs
-// 64 and 161 vs 155).
+// Whether the rows run on the tiled int8 product: where it is the fastest
+// kernel, unless a prefill GEMM family is asked for by number.
+static bool use_i8t(uint32_t type, int M, int K, int N) {
+    return i8t_preferred(type, M, K, N) && !(forced_gemm_kernel() && gemm_supported(type, M, K));
+}
+
+// Whether M > 16 rows run on the fp16/fp8 GEMM (Q4_K).
 static bool use_gemm(uint32_t type, int M, int K, int N, const uint8_t* w) {
-    if (!gemm_supported(type, M, K) || i8mf_supported(type, M, K, N, w)) return false;
+    if (!gemm_supported(type, M, K) || i8mf_supported(type, M, K, N, w) || use_i8t(type, M, K, N)) return false;
+    // small row counts run faster as 16-row chunks on the small-M int8 kernel
+    // than on the GEMM's 64-token tiles (measured per call at N x K = 14336 x
+    // 4096 / 4096 x 14336: M=17 32 vs 49 and 52 vs 136 us; M=32 49 vs 54 and
+    // 82 vs 142)
     if (type == T_Q4_K && i8mf_supported(type, 16, K, N, w) && (M <= 32 || (M <= 64 && N <= 4096))) return false;
     return true;
 }
 
 static int gemm_q(const ActView& A, void* planes, const uint8_t* w, uint32_t type, float* y,
                   int M, int K, int N, hipStream_t st) {
+    if (use_i8t(type, M, K, N)) {
+        LP_HIP(launch_gemm_i8t(type, w, A, y, M, K, N, st));
+        return LP_OK;
+    }
     if (i8mf_supported(type, M, K, N, w)) {
         LP_HIP(launch_gemv_i8mf(type, w, A, y, M, K, N, st));
         return LP_OK;
@@ -193,22 +202,8 @@ static int gemm_q(const ActView& A, void* planes, const uint8_t* w, uint32_t typ
         LP_HIP(launch_gemm(type, w, A, planes, y, M, K, N, st));
         return LP_OK;
     }
-    // no GEMM kernel for the type: chunks of rows through the widest small-M
-    // path (Q8_0: several 16-token tiles per workgroup; 16 rows on int8 MFMA
-    // where the type has it, else 8 on the GEMV)
-    if (M > 16 && i8_chunk_supported(type, K, N, w)) {
-        const int ch = i8_chunk_rows();
-        for (int m0 = 0; m0 < M; m0 += ch) {
-            const int mt = M - m0 < ch ? M - m0 : ch;
-            ActView sub = A;
-            sub.qs = A.qs + (size_t)m0 * K;
-            sub.d = A.d + (size_t)m0 * (K / 32);
-            sub.sum = A.sum + (size_t)m0 * (K / 32);
-            sub.s16 = A.s16 + (size_t)m0 * (K / 32);
-            LP_HIP(launch_i8_chunk(type, w, sub, y + (size_t)m0 * N, mt, K, N, st));
-        }
-        return LP_OK;
-    }
+    // chunks of rows through the widest small-M path: 16 rows on int8 MFMA
+    // where the type has it, else 8 on the GEMV
     const int chunk = i8mf_supported(type, 16, K, N, w) ? 16 : 8;
     for (int m0 = 0; m0 < M; m0 += chunk) {
         const int mt = M - m0 < chunk ? M - m0 : chunk;
@@ -226,10 +221,10 @@ static int gemm_q(const ActView& A, void* planes, const uint8_t* w, uint32_t typ
 // The kernel gemm_q runs for these operands (first chunk when rows are
 // chunked), for the routing probe lp_gemm_route.
 static const char* gemm_q_route(uint32_t type, int M, int K, int N, const uint8_t* w) {
+    if (use_i8t(type, M, K, N)) return "i8mf";
     if (i8mf_supported(type, M, K, N, w))
         return rq_preferred(type, M, K, N, w) ? "rq" : q6rq_preferred(type, M, K, N, w) ? "q6rq" : "i8mf";
     if (use_gemm(type, M, K, N, w)) return "gemm";
-    if (M > 16 && i8_chunk_supported(type, K, N, w)) return "i8mf";
     const int chunk = i8mf_supported(type, 16, K, N, w) ? 16 : 8;
     const int mt = M < chunk ? M : chunk;
     if (i8mf_supported(type, mt, K, N, w))
@@ -393,10 +388,6 @@ static int host_gemm(const float* x, const uint8_t* w, uint32_t type, float* y, 
         LP_HIP(launch_gemv_fact(type, wd, c->xd, c->yd, M, K, N, c->stream));
     } else if (gemv_fused_supported(type, M, K, wd)) {
         LP_HIP(launch_gemv_fused(type, wd, c->xd, c->yd, M, K, N, c->stream));
-    } else if (i8mf_supported(type, M, K, N, wd)) {
-        const ActView A = ws_view_full(c->ws, M, K);
-        LP_HIP(launch_quantize(c->xd, M, K, A, c->stream));
-        LP_HIP(launch_gemv_i8mf(type, wd, A, c->yd, M, K, N, c->stream));
     } else if (use_gemm(type, M, K, N, wd) && !gemm_i8_preferred(type, M, K, N)) {
         void* planes = ws_planes(c->ws, M, K);
         LP_HIP(launch_planes_from_x(c->xd, planes, M, K, c->stream, N, c->yd));

@@ -744,9 +744,6 @@ quant_planes_kernel(const float* __restrict__ x, int K, Planes P, float* __restr
 
 constexpr int kMfWaves = 8;
 constexpr int kMfTiles = 2;         // 16-row tiles per workgroup (every wave takes all of them)
-constexpr int kI8ChunkTt = 2;      // Q8_0 / Q6_K prefill chunks: 16-token tiles per workgroup
-constexpr bool kQ6Chunk = true;
-constexpr bool kQ40Chunk = true;
 constexpr int kMfMoeWaves = 2;      // grouped MoE: waves per workgroup
 constexpr int kMfMoeRows = 64;    // grouped MoE: weight rows per workgroup (at least two sets)
 constexpr int kMfMaxM = 16;
@@ -1157,110 +1154,6 @@ gemv_q6k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restri
     }
 }
 
-// Q8_0 for 9 <= M <= 16 on the same int8 MFMA: one 32-element block per
-// instruction, B = the int8 codes, epilogue acc += P * (xd * fp16(d))
-// (dot_row_q8_0_int_neon, src/matmul_simd.cpp:143-160). Waves take K-slices
-// of 8-block groups; the 34-byte blocks are 2-byte aligned.
-// TT 16-token tiles per workgroup (M <= 16 TT): each weight fragment feeds
-// TT MFMAs, so prefill chunks of 32-64 rows read the weights once per chunk.
-template <uint32_t T, int TL, int NWV, int TT = 1>
-__global__ void __launch_bounds__(64 * NWV)
-gemv_b32_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restrict__ y, int M, int K, int N) {
-    static_assert(T == T_Q8_0 || T == T_Q4_0, "Q8_0 / Q4_0");
-    static_assert(TL * TT <= NWV, "one wave per output tile in the final sum");
-    constexpr int BPB = T == T_Q8_0 ? 34 : 18;
-    constexpr int TK = 16 * TT;
-    __shared__ f4v red[NWV][TL * TT][64];
-    extern __shared__ __attribute__((aligned(16))) float sdx[];   // [nb][TK] xd
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int tok = lane & 15, g = lane >> 4;
-    const int nb = K >> 5, ngr = K >> 8;
-    for (int i = threadIdx.x; i < nb * TK; i += blockDim.x) {
-        const int b = i / TK, t = i % TK;
-        sdx[i] = t < M ? A.d[(size_t)t * nb + b] : 0.0f;
-    }
-    __syncthreads();
-    bool tv[TT];
-    const int8_t* aq[TT];
-#pragma unroll
-    for (int u = 0; u < TT; u++) {
-        tv[u] = tok + 16 * u < M;
-        aq[u] = A.qs + (size_t)(tv[u] ? tok + 16 * u : 0) * K + 8 * g;
-    }
-    const int row0 = blockIdx.x * (16 * TL) + (lane & 15);
-    const int gr0 = wv * ngr / NWV, gr1 = (wv + 1) * ngr / NWV;
-    const uint8_t* wr[TL];
-#pragma unroll
-    for (int t = 0; t < TL; t++) {
-        int row = row0 + 16 * t;
-        row = row < N ? row : N - 1;
-        wr[t] = w + (size_t)row * rb;
-    }
-    const i4v zi = {0, 0, 0, 0};
-    const f4v z4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    f4v acc[TL][TT];
-#pragma unroll
-    for (int t = 0; t < TL; t++)
-#pragma unroll
-        for (int u = 0; u < TT; u++) acc[t][u] = z4;
-    for (int gr = gr0; gr < gr1; gr++) {
-        long av[TT][8];
-#pragma unroll
-        for (int u = 0; u < TT; u++)
-#pragma unroll
-            for (int b = 0; b < 8; b++)
-                av[u][b] = tv[u] ? *reinterpret_cast<const long*>(aq[u] + 32 * (8 * gr + b)) : 0L;
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const int kb = 8 * gr + b;
-#pragma unroll
-            for (int t = 0; t < TL; t++) {
-                const uint8_t* blk = wr[t] + (size_t)kb * BPB;
-                const float d = fp16_bits_to_f32(*reinterpret_cast<const uint16_t*>(blk));
-                uint2 c;
-                if constexpr (T == T_Q8_0) {
-                    c = ld8_a2(blk + 2 + 8 * g);
-                } else {
-                    // elements 8g..8g+7: low nibbles of bytes 8g.. (g < 2), high
-                    // nibbles of bytes 8(g - 2).. ; code - 8 per byte (no borrow)
-                    const uint2 r = ld8_a2(blk + 2 + 8 * (g & 1));
-                    const int sh = g < 2 ? 0 : 4;
-                    c.x = ((((r.x >> sh) & 0x0f0f0f0fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-                    c.y = ((((r.y >> sh) & 0x0f0f0f0fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-                }
-                const long bw = (long)((unsigned long)c.x | ((unsigned long)c.y << 32));
-#pragma unroll
-                for (int u = 0; u < TT; u++) {
-                    const f4v xd = *reinterpret_cast<const f4v*>(sdx + (size_t)kb * TK + 16 * u + 4 * g);
-                    const i4v S = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[u][b], bw, zi, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[t][u][r] = fmaf(d * xd[r], (float)S[r], acc[t][u][r]);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < TL; t++)
-#pragma unroll
-        for (int u = 0; u < TT; u++) red[wv][t * TT + u][lane] = acc[t][u];
-    __syncthreads();
-    // wave i sums output tile i (row tile i / TT, token tile i % TT)
-    if (wv < TL * TT) {
-        const int t = wv / TT, u = wv % TT;
-        f4v sum = red[0][wv][lane];
-#pragma unroll
-        for (int i = 1; i < NWV; i++) sum += red[i][wv][lane];
-        const int row = row0 + 16 * t;
-        if (row < N) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int tt = 16 * u + 4 * g + r;
-                if (tt < M) y[(size_t)tt * N + row] = sum[r];
-            }
-        }
-    }
-}
-
 bool i8mf_supported(uint32_t type, int M, int K, int N, const uint8_t* w) {
     // LDS: per block and token the scale (Q4_K also the sum), at most 64 KiB
     if (M > kMfMaxM || K % 256 != 0) return false;
@@ -1273,46 +1166,7 @@ bool i8mf_supported(uint32_t type, int M, int K, int N, const uint8_t* w) {
         return M >= min_m && (size_t)(K / 32) * 16 * 8 <= 64 * 1024 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
     }
     if (M < kMfMinM) return false;
-    // Q8_0 from 9 rows (measured at 14336 x 4096: M=8 64 us vs 54 on the GEMV,
-    // M=16 70 vs 104, M=64 266 vs 392); Q4_0 was no faster than the GEMV
-    const bool lds_ok = (size_t)(K / 32) * 16 * 4 <= 64 * 1024 && reinterpret_cast<uintptr_t>(w) % 2 == 0;
-    if (type == T_Q6_K) return lds_ok;
-    if (type == T_Q8_0) return M >= 9 && lds_ok;
-    return false;
-}
-
-// Q8_0, Q4_0 and Q6_K prefill rows in chunks of kI8ChunkTt * 16 tokens
-// (one weight pass per chunk), 32-row workgroups of 8 waves; Q6_K only where
-// those fill 1.5 rounds of CUs: 1 <= M <= 16 * kI8ChunkTt. Measured (us per
-// call), Q8_0 against 16-row chunks: 14336x4096 M = 32 / 64 / 256 113 / 223
-// / 884 -> 67 / 132 / 522, 4096x4096 M=128 142 -> 134 (16-row workgroups of
-// 16 waves there: 151); Q4_0 against 8-row GEMV chunks: 14336x4096 M=64 262
-// -> 130, 4096x4096 M=128 193 -> 131, 1024x4096 M=64 72.5 -> 65; Q6_K
-// 14336x4096 M=64 156 -> 100, but 4096x4096 M=128 97.5 -> 111 (so not
-// there); four token tiles slower everywhere (Q8_0 14336x4096 M=256 948)
-bool i8_chunk_supported(uint32_t type, int K, int N, const uint8_t* w) {
-    return (type == T_Q8_0 || (type == T_Q6_K && kQ6Chunk) || (type == T_Q4_0 && kQ40Chunk)) && K % 256 == 0 &&
-           (size_t)(K / 32) * 16 * kI8ChunkTt * 4 <= 64 * 1024 && reinterpret_cast<uintptr_t>(w) % 2 == 0 &&
-           (2 * ((N + 31) / 32) >= 3 * device_cu_count() || type != T_Q6_K);
-}
-int i8_chunk_rows() { return 16 * kI8ChunkTt; }
-
-hipError_t launch_i8_chunk(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
-                            hipStream_t st) {
-    if (M <= 0 || N <= 0) return hipSuccess;
-    if (M > 16 * kI8ChunkTt || !i8_chunk_supported(type, K, N, w)) return hipErrorInvalidValue;
-    constexpr int TT = kI8ChunkTt;
-    const size_t shm = (size_t)(K / 32) * 16 * TT * 4;
-    const long rbq = (long)row_bytes(type, K);
-    if (type == T_Q6_K)
-        hipLaunchKernelGGL((gemv_q6k_i8mf<2, 8, TT>), dim3((N + 31) / 32), dim3(512), shm, st, w, rbq, A, y, M, K, N);
-    else if (type == T_Q4_0)
-        hipLaunchKernelGGL((gemv_b32_i8mf<T_Q4_0, 2, 8, TT>), dim3((N + 31) / 32), dim3(512), shm, st, w, rbq, A, y,
-                           M, K, N);
-    else
-        hipLaunchKernelGGL((gemv_b32_i8mf<T_Q8_0, 2, 8, TT>), dim3((N + 31) / 32), dim3(512), shm, st, w, rbq, A, y,
-                           M, K, N);
-    return hipGetLastError();
+    return type == T_Q6_K && (size_t)(K / 32) * 16 * 4 <= 64 * 1024 && reinterpret_cast<uintptr_t>(w) % 2 == 0;
 }
 
 hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
@@ -1322,16 +1176,6 @@ hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, f
     if (rq_preferred(type, M, K, N, w)) return launch_gemv_rq(w, A, y, M, K, N, st);
     if (q6rq_preferred(type, M, K, N, w)) return launch_gemv_q6rq(w, A, y, M, K, N, st);
     const dim3 grid((N + 16 * kMfTiles - 1) / (16 * kMfTiles));
-    if (type == T_Q8_0) {
-        const size_t shm = (size_t)(K / 32) * 16 * 4;
-        const long rbq = (long)row_bytes(type, K);
-        if (2 * ((N + 31) / 32) >= 3 * device_cu_count())
-            hipLaunchKernelGGL((gemv_b32_i8mf<T_Q8_0, 2, 8>), grid, dim3(512), shm, st, w, rbq, A, y, M, K, N);
-        else
-            hipLaunchKernelGGL((gemv_b32_i8mf<T_Q8_0, 1, 16>), dim3((N + 15) / 16), dim3(1024), shm, st, w, rbq, A, y,
-                               M, K, N);
-        return hipGetLastError();
-    }
     if (type == T_Q6_K) {
         // few weight rows (e.g. a down projection, 3584 rows of K 18944): 16-row
         // workgroups of 16 waves, so the K-slices spread over twice the CUs.
@@ -1385,6 +1229,7 @@ size_t gemm_planes_bytes(int M, int K) {
 // fragment-order planes (gemm_q4k_wt) with 128 x 256 and 256 x 256 tiles.
 static int g_gemm_kernel = 0;
 void set_gemm_kernel(int k) { g_gemm_kernel = k; }
+int forced_gemm_kernel() { return g_gemm_kernel; }
 
 bool gemm_i8_preferred(uint32_t type, int M, int K, int N) {
     return g_gemm_kernel == 3 && gemm_i8_supported(type, M, K) && N > 0;

@@ -91,15 +91,13 @@ hipError_t launch_gemv_fused_batch(const uint8_t* const* w, float* const* y, con
 // M <= 16 on the small-M MFMA kernel, larger M on the tiled GEMM.
 bool gemm_supported(uint32_t type, int M, int K);
 // Small M on int8 MFMA straight from the quantized blocks (no planes):
-// Q4_K and Q6_K for 5 <= M <= 16 (Q4_K from M = 3 when N < 32 x CUs and K >= 14336),
-// Q8_0 for 9 <= M <= 16.
+// Q4_K and Q6_K for 5 <= M <= 16 (Q4_K from M = 3 when N < 32 x CUs and K >= 14336).
 bool i8mf_supported(uint32_t type, int M, int K, int N, const uint8_t* w);
-// Q8_0 / Q6_K rows beyond 16 in chunks of i8_chunk_rows() on the int8 MFMA
-// kernels with several token tiles per workgroup (lp_gemm.hip).
-bool i8_chunk_supported(uint32_t type, int K, int N, const uint8_t* w);
-int i8_chunk_rows();
-hipError_t launch_i8_chunk(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
-                            hipStream_t st);
+// Tiled int8 MFMA product of the quantized blocks (lp_gemm_i8t.hip) for all five
+// int8 types; i8t_preferred: the shapes where it is the fastest kernel.
+bool i8t_preferred(uint32_t type, int M, int K, int N);
+hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
+                           hipStream_t st);
 hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
                             hipStream_t st);
 // Q4_K for 1 <= M <= 8 on 4x4 int8 MFMA blocks, a row quad per wave
@@ -126,6 +124,7 @@ bool gemm_i8_supported(uint32_t type, int M, int K);
 bool gemm_i8_preferred(uint32_t type, int M, int K, int N);
 // Prefill GEMM kernel family (0 by shape, 1 split-precision, 2 fragment-order, 3 int8, 4/5 wide-token 128/256-token tiles).
 void set_gemm_kernel(int k);
+int forced_gemm_kernel();
 hipError_t launch_gemm_i8(const uint8_t* w, const ActView& A, void* planes, float* y, int M, int K, int N,
                           hipStream_t st);
 bool gemm_fr_supported(uint32_t type, int M, int K);

@@ -1,0 +1,79 @@
+"""The tiled int8 MFMA product (Q8_0, Q4_0, Q5_0, Q6_K and Q4_K rows beyond the
+small-M kernels) at the edges of its tiles and forms, against the oracle."""
+import numpy as np
+import pytest
+
+from hip_util import L, gemm_dev, normwise, synth_weights, synth_x, to_dev
+from oracle.oracle import Q4_0, Q4_K, Q5_0, Q6_K, Q8_0
+
+pytestmark = pytest.mark.gpu
+NAMES = {Q8_0: "Q8_0", Q4_0: "Q4_0", Q5_0: "Q5_0", Q6_K: "Q6_K", Q4_K: "Q4_K"}
+
+# Integer block sums are exact on both sides. Each side rounds the scale product
+# and the additions of a chain: at most ~(K/32 + 3) half-ulps of the largest
+# partial sum, K <= 2048 here: 67 * 2^-25 = 2e-6 normwise, and twice that for two
+# sides.
+TOL = 4e-6
+
+# (M, N, K): one token and one row past a 32- and 64-tile, K ending inside a
+# 128-element stage (64-, 32- and 192-element tails), single-stage K, one stage
+# pair and its neighbours, M and N that take each form (32x32 with 8 and 4 K
+# groups, 64x64 with 2 and 1, 128x128)
+SHAPES32 = [(5, 31, 64), (8, 33, 192), (17, 1, 1088), (33, 65, 448), (65, 127, 2048)]
+SHAPES256 = [(17, 33, 256), (33, 31, 512), (65, 129, 1280), (127, 64, 2048)]
+FORMS = [(31, 8200, 256), (40, 8200, 512), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256)]
+CASES = ([(t, *s) for t in (Q8_0, Q4_0) for s in SHAPES32] + [(Q5_0, M, N, K + 32 * (K < 2048)) for M, N, K in SHAPES32]
+         + [(Q6_K, *s) for s in SHAPES256] + [(t, *s) for t in NAMES if t != Q4_K for s in FORMS]
+         + [(Q4_K, *s) for s in ((65, 129, 1280), (127, 64, 2048), (33, 8200, 512), (96, 14400, 256), (130, 16300, 256))])
+
+
+def weights(t, K, N, seed):
+    w = synth_weights(t, K, N, seed=seed)
+    if t == Q5_0:                                          # finite block scales
+        d = np.abs(np.random.default_rng(seed).standard_normal(w.size // 22)) * 0.01
+        w.reshape(-1, 22)[:, 0:2] = d.astype(np.float16).view(np.uint8).reshape(-1, 2)
+    return w
+
+
+@pytest.mark.parametrize("t,M,N,K", CASES, ids=[f"{NAMES[c[0]]}-{c[1]}x{c[2]}x{c[3]}" for c in CASES])
+def test_i8t_matches_oracle(orc, t, M, N, K):
+    print(f"i8t {NAMES[t]} M={M} N={N} K={K}", flush=True)
+    w = weights(t, K, N, seed=M + N + K + t)
+    assert L().lp_gemm_route(t, M, K, N, to_dev(w).data_ptr()).decode() == "i8mf"
+    x = synth_x(M, K, seed=M + 1, outliers=0.01)
+    x[M // 2, :32] = 0.0                                   # a block of zeros
+    y = gemm_dev(t, x, w, N)
+    rows = np.unique(np.linspace(0, N - 1, 48).astype(int))   # both ends and between
+    rb = len(w) // N
+    ref = orc.gemm_int(t, x, np.concatenate([w[r * rb:(r + 1) * rb] for r in rows]), len(rows))
+    assert normwise(y[:, rows], ref) <= TOL
+
+
+@pytest.mark.parametrize("t", list(NAMES), ids=list(NAMES.values()))
+def test_i8t_rows_do_not_depend_on_their_neighbours(orc, t):
+    """Every form adds the same 256-element chains in 64 bits, so the first 70
+    rows of calls that run on different forms are the same numbers."""
+    K, N = 1024, 3000
+    w = weights(t, K, N, seed=9 + t)
+    x = synth_x(700, K, seed=10, outliers=0.01)
+    first = gemm_dev(t, x[:70], w, N)
+    for M in (129, 300, 700):
+        y = gemm_dev(t, x[:M], w, N)
+        assert np.array_equal(y[:70].view(np.uint32), first.view(np.uint32)), M
+
+
+@pytest.mark.parametrize("t", list(NAMES), ids=list(NAMES.values()))
+def test_i8t_non_finite_rows(orc, t):
+    """A NaN or infinity in a row makes that row NaN as the reference's scale
+    does, and leaves the others alone."""
+    K, N, M = 512, 96, 70
+    w = weights(t, K, N, seed=20 + t)
+    x = synth_x(M, K, seed=21)
+    x[3, 40] = np.nan
+    x[69, 511] = np.inf
+    x[68, 0] = -np.inf
+    y = gemm_dev(t, x, w, N)
+    ref = orc.gemm_int(t, x, w, N)
+    assert np.array_equal(np.isnan(y), np.isnan(ref))
+    good = [m for m in range(M) if m not in (3, 68, 69)]
+    assert normwise(y[good], ref[good]) <= TOL
