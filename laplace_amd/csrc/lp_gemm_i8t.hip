@@ -557,38 +557,41 @@ gemm_i8t(I8tArgs g) {
     for (int it = 0; it < iters; it++) {
         const int s = 2 * (it * WK + kg);
         stage(Flag<true>{}, s + 1);
+        // few stages per group: the last one does not wait for a load nobody needs
+        // (the same call 11.6 -> 11.0 us)
+        if (WK > 1 && it == iters - 1) {
+            compute(Flag<false>{}, lds + (NBUF == 1 ? 0 : L::bytes));
+            flush();
+            break;
+        }
         stage(Flag<false>{}, s + 2 * WK);
         flush();
     }
     if constexpr (WK > 1) {
         if constexpr (NBUF == 1) __syncthreads();      // every group is done with its buffer
-        // groups 1.. leave their sums in LDS, group 0 adds them in order
-        double* red = reinterpret_cast<double*>(smem);
-        constexpr int kPer = MT * NT * 16 * 64;        // sums of one wave
+        // All groups leave their sums in LDS; group kg adds those of registers kg,
+        // kg + WK, .. in the groups' order (against one group adding the others' one
+        // after the other: Q8_0 N 4096 K 4096 M 16 13.1 -> 11.6 us with the quantizer).
+        double* red = reinterpret_cast<double*>(smem) + wave * MT * NT * 16 * 64 + lane;
+        constexpr int kGrp = WM * WN * MT * NT * 16 * 64;
 #pragma unroll
-        for (int q = 1; q < WK; q++) {
-            if (kg == q) {
+        for (int t = 0; t < MT; t++)
 #pragma unroll
-                for (int t = 0; t < MT; t++)
+            for (int r = 0; r < NT; r++)
 #pragma unroll
-                    for (int r = 0; r < NT; r++)
+                for (int i = 0; i < 16; i++) red[kg * kGrp + ((t * NT + r) * 16 + i) * 64] = sum[t][r][i];
+        __syncthreads();
+        for (int j = kg; j < MT * NT * 16; j += WK) {
+            double u = red[j * 64];
 #pragma unroll
-                        for (int i = 0; i < 16; i++)
-                            red[wave * kPer + ((t * NT + r) * 16 + i) * 64 + lane] = sum[t][r][i];
+            for (int q = 1; q < WK; q++) u += red[q * kGrp + j * 64];
+            const int i = j & 15, n = n0 + (wn * NT + (j >> 4) % NT) * 32 + col;
+            const int m = m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+            if (m < g.M && n < g.N) {
+                g.y[(size_t)m * g.N + n] = (float)u;
             }
-            __syncthreads();
-            if (kg == 0) {
-#pragma unroll
-                for (int t = 0; t < MT; t++)
-#pragma unroll
-                    for (int r = 0; r < NT; r++)
-#pragma unroll
-                        for (int i = 0; i < 16; i++)
-                            sum[t][r][i] += red[wave * kPer + ((t * NT + r) * 16 + i) * 64 + lane];
-            }
-            __syncthreads();
         }
-        if (kg != 0) return;
+        return;
     }
 #pragma unroll
     for (int r = 0; r < NT; r++) {
@@ -606,7 +609,7 @@ gemm_i8t(I8tArgs g) {
 template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
 hipError_t launch_cfg(I8tArgs g, hipStream_t st) {
     constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
-    constexpr int red = WK > 1 ? WM * WN * MT * NT * 8192 : 0;
+    constexpr int red = WK > 1 ? WK * WM * WN * MT * NT * 8192 : 0;
     constexpr int bufs = WK * (WM * WN == 1 ? 1 : 2) * Lay<T, BM, BN>::bytes;
     constexpr int lds = bufs > red ? bufs : red;
     static_assert(lds <= 160 * 1024, "LDS");
@@ -667,13 +670,19 @@ hipError_t launch_t(const I8tArgs& g, Form f, hipStream_t st) {
 }
 }  // namespace
 
-// Where this kernel is the fastest one (M >= 5 rows; weights aligned as the
-// entry points check). Against the small-M kernels it replaces (us, M 8 / 16 of
-// N 14336 K 4096): Q8_0 48.8 / 54.9 -> 16.1 / 17.0, Q4_0 34.6 / 65.8 -> 15.4,
-// Q5_0 35.3 / 69.0 -> 18.9; at M <= 4 their GEMVs are as fast. Q6_K from 9 rows
-// where 32-row tiles fill the CUs (N 14336 M 9 37.0 -> 20.6), else from 13 (N 4096
-// M 12 12.7 against 13.2 here, M 16 13.9 -> 13.1, M 17 18.5 -> 12.9, M 512 382 -> 65; N 3584 K 18944 M 512 1327
-// -> 270).
+// Where this kernel is the fastest one (weights aligned as the entry points check).
+// Up to 32 rows its time depends on K alone (8 to 12 us with the quantizer), a GEMV's
+// on N too: up to 8 rows the line is a number of outputs. Measured (us, GEMV against
+// this): Q8_0 K 4096: N 1024 M 8 9.9 / 11.3, N 2048 M 5 9.9 / 11.2, N 4096 M 5 13.6 /
+// 10.9, M 8 19.2 / 10.8; K 1024 N 4096 M 5 7.9 / 8.7, M 8 9.9 / 8.2; Q4_0 N 2048 M 5
+// 9.4 / 11.0, N 4096 M 5 11.6 / 10.3; Q5_0 N 2048 M 8 11.1 / 13.6, N 4096 M 8 13.5 /
+// 12.4. Beyond 8 rows their GEMVs run twice (N 14336 K 4096 M 16: Q4_0 65.8 -> 15.4,
+// Q5_0 69 -> 18.9; Q8_0's 16-row kernel 54.9 -> 17.0; N 1024 K 1024 8.5 -> 8.3).
+// Q6_K from 9 rows where 32-row tiles fill the CUs (N 14336 M 9 37.0 -> 20.6), else
+// from 13 (K 4096, N 512 .. 4096: M 13 13.8 -> 13.2, M 17 18.8 -> 13.3, N 4096 M 512
+// 382 -> 65; N 3584 K 18944 M 512 1327 -> 270). Short rows (K 1024: M 16 8.5 against
+// 9.8 here, M 17 12.8 -> 9.9) stay there up to 15 rows, and 16 below K = 1024: from
+// there on, 16 rows give the bits of the first 16 of a longer prompt.
 // Q4_K where the 16-row chunks of the small-M kernel end (beyond 32 rows, 64 for
 // up to 4096 weight rows) while one round of 128 x 128 tiles covers the product,
 // and for K > 4096 not where that round would be half empty (N 14336 M 64 42 -> 27,
@@ -683,8 +692,9 @@ hipError_t launch_t(const I8tArgs& g, Form f, hipStream_t st) {
 bool i8t_preferred(uint32_t type, int M, int K, int N) {
     const long cus = device_cu_count();
     switch (type) {
-        case T_Q8_0: case T_Q4_0: case T_Q5_0: return M >= 5;
-        case T_Q6_K: return M >= 13 || (M >= 9 && (N + 31) / 32 > cus);
+        case T_Q8_0: case T_Q4_0: case T_Q5_0:
+            return M > 8 || (M >= 5 && (long)M * N >= (type == T_Q5_0 || K < 2048 ? 32768 : 20000));
+        case T_Q6_K: return M > 16 || (M >= (K < 2048 ? 16 : 13) && K >= 1024) || (M >= 9 && (N + 31) / 32 > cus);
         case T_Q4_K: {
             if (M <= 32 || (M <= 64 && N <= 4096)) return false;
             const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 127) / 128);

@@ -19,7 +19,7 @@ TOL = 4e-6
 # 128-element stage (64-, 32- and 192-element tails), single-stage K, one stage
 # pair and its neighbours, M and N that take each form (32x32 with 8 and 4 K
 # groups, 64x64 with 2 and 1, 128x128)
-SHAPES32 = [(5, 31, 64), (8, 33, 192), (17, 1, 1088), (33, 65, 448), (65, 127, 2048)]
+SHAPES32 = [(9, 31, 64), (12, 33, 192), (17, 1, 1088), (33, 65, 448), (65, 127, 2048), (5, 6555, 1088)]
 SHAPES256 = [(17, 33, 256), (33, 31, 512), (65, 129, 1280), (127, 64, 2048)]
 FORMS = [(31, 8200, 256), (40, 8200, 512), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256)]
 CASES = ([(t, *s) for t in (Q8_0, Q4_0) for s in SHAPES32] + [(Q5_0, M, N, K + 32 * (K < 2048)) for M, N, K in SHAPES32]
