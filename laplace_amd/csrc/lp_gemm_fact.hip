@@ -1,0 +1,643 @@
+// lp_gemm_fact.hip - tiled bf16-MFMA product of fp32 activation rows with F32 /
+// F16 / BF16 / Q2_K / Q3_K / Q5_K weights (prompt rows), at fp32 precision.
+//
+// These types multiply fp32 activations (dot_row_f32 .. dot_row_q5_k,
+// src/matmul.cpp:63-314). The matrix unit's fp32 products run at a sixteenth of
+// its bf16 rate, so an fp32 value is split into the three bf16 pieces it is the
+// exact sum of, x = x1 + x2 + x3, and multiplied piece by piece with fp32
+// accumulation:
+//   BF16        w is one piece:             3 products
+//   Q2_K, Q3_K  scale times code (<= 45, <= 128) is a bf16 value; d once per 256
+//   Q5_K        the 5-bit code is one; d * scale once per 32 (on the VALU)
+//   F16         w = w1 + w2 (8 + 3 bits):   5 products (x3 w2 is below 2^-24)
+//   F32         w = w1 + w2 + w3:           6 products (the rest below 2^-24)
+// The min terms of Q2_K / Q5_K (-dmin * m * sum x) take the sums of x per 16 / 32
+// elements, split the same way, in one small product per 32 elements. Every 64
+// elements the fp32 accumulators are added to 64-bit sums, so the result is nearer
+// to the exact product than the fp32 dots of the GEMV kernels are.
+//
+// Work split: that of the int8 product (lp_gemm_i8t.hip). A stage is 64 elements:
+// the activation tile is split and the weight tile decoded once per workgroup into
+// LDS in operand order ([32 rows][16 k][half][row][8 bf16]); the next stage is in
+// registers meanwhile.
+//
+// What bounds it (BF16, N 4096 K 4096 M 512, 95 us of which ~7 launch: 540 TFLOP/s of
+// bf16 products, the GEMVs 1205 us, one pass over the weights per 4 rows): loads are
+// hidden behind the products; splitting x and writing its planes (58 us alone) and the
+// products (72 - 80 us alone) follow each other in every wave. Large: M 2048 N 14336
+// 15890 -> 928 us, Q5_K N 4096 K 14336 M 2048 95144 -> 1253. Normwise errors against
+// 64-bit sums 5e-8 .. 1e-7, the GEMVs' 0.7e-7 .. 3e-7.
+#include <hip/hip_runtime.h>
+
+#include "lp_dequant_one.h"
+#include "lp_internal.h"
+
+namespace lp {
+namespace {
+
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
+typedef short s4v __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+constexpr int kH = 528;                  // 32 rows x 16 B, padded: the 8 pieces of a row written together hit distinct banks
+constexpr int kTile = 8 * kH;            // 32 rows x 64 elements of one plane
+
+struct FactArgs {
+    const uint8_t* w;
+    const float* x;
+    float* y;
+    int M, N, K;
+    size_t rb;
+    int ntm, ntn;
+};
+
+template <uint32_t T>
+struct Traits {
+    static constexpr int kPlanes = T == T_F32 ? 3 : T == T_F16 ? 2 : 1;    // bf16 pieces of a weight
+    static constexpr bool kQuant = T == T_Q2_K || T == T_Q3_K || T == T_Q5_K;
+    static constexpr bool kMin = T == T_Q2_K || T == T_Q5_K;
+    // staging tasks per row: 4 values of F32, 8 of F16 / BF16, 8 code bytes (16 values) of the others
+    static constexpr int kTasks = T == T_F32 ? 16 : kQuant ? 4 : 8;
+    // floats per row and stage: Q5_K d * scale x 2, m x 2, dmin; Q3_K d; Q2_K d, dmin, m x 4
+    static constexpr int kScales = T == T_Q5_K ? 5 : T == T_Q2_K ? 6 : T == T_Q3_K ? 1 : 0;
+};
+
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {      // rounded to nearest even
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
+}
+__device__ __forceinline__ float lo_f32(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float hi_f32(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
+__device__ __forceinline__ float hi16(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
+
+// v[4] as PL planes of 4 bf16 whose sum is v: each piece is the rest rounded to
+// nearest. Values whose first piece would round to infinity, and infinities
+// (their own first piece), are cut off instead.
+template <int PL>
+__device__ __forceinline__ void split4(const float (&v)[4], u32x2 (&o)[PL]) {
+    float r[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        o[0][i] = pk_bf16(v[2 * i], v[2 * i + 1]);
+        r[2 * i] = v[2 * i] - lo_f32(o[0][i]);
+        r[2 * i + 1] = v[2 * i + 1] - hi_f32(o[0][i]);
+        if constexpr (PL > 1) o[1][i] = pk_bf16(r[2 * i], r[2 * i + 1]);
+        if constexpr (PL > 2)
+            o[2][i] = pk_bf16(r[2 * i] - lo_f32(o[1][i]), r[2 * i + 1] - hi_f32(o[1][i]));
+    }
+    if (PL > 1 && fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))) >= 0x1.fe8p127f) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            uint32_t q[2][3];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float x = v[2 * i + k], x1 = hi16(x), r1 = fabsf(x) == __builtin_inff() ? 0.0f : x - x1;
+                const float x2 = hi16(r1);
+                q[k][0] = __float_as_uint(x1) >> 16;
+                q[k][1] = __float_as_uint(x2) >> 16;
+                q[k][2] = __float_as_uint(r1 - x2) >> 16;
+            }
+#pragma unroll
+            for (int p = 0; p < PL; p++) o[p][i] = q[0][p] | (q[1][p] << 16);
+        }
+    }
+}
+
+template <uint32_t T>
+struct WReg {
+    u32x4 a;             // F32: 4 values; F16, BF16: 8
+    u32x2 q, h;          // code bytes, high-bit bytes
+    u32x4 hd;            // Q5_K header
+    uint32_t s0, s1, d;  // scale bytes, d (and dmin)
+};
+
+// Task t of the 64-element stage s of the row at base + off. F32, F16, BF16: past
+// the row's end its last bytes again.
+template <uint32_t T>
+__device__ __forceinline__ void w_load(WReg<T>& r, const uint8_t* base, uint32_t off, uint32_t rb, int s, int t) {
+    if constexpr (T == T_F32 || T == T_F16 || T == T_BF16) {
+        uint32_t o = (uint32_t)s * (T == T_F32 ? 256u : 128u) + 16u * t;
+        o = off + (o < rb - 16 ? o : rb - 16);
+        if constexpr (T == T_F32) r.a = *reinterpret_cast<const u32x4_a4*>(base + o);
+        else r.a = *reinterpret_cast<const u32x4_a2*>(base + o);
+    } else if constexpr (T == T_Q5_K) {
+        const uint8_t* sb = base + (size_t)(s >> 2) * 176;
+        r.hd = *reinterpret_cast<const u32x4_a4*>(sb + off);
+        r.h = *reinterpret_cast<const u32x2_a2*>(sb + 16 + (off + 8u * t));
+        r.q = *reinterpret_cast<const u32x2_a2*>(sb + 48 + 32 * (s & 3) + (off + 8u * t));
+    } else if constexpr (T == T_Q3_K) {
+        const uint8_t* sb = base + (size_t)(s >> 2) * 110;
+        r.h = *reinterpret_cast<const u32x2_a2*>(sb + (off + 8u * t));
+        r.q = *reinterpret_cast<const u32x2_a2*>(sb + 32 + 32 * ((s & 3) >> 1) + (off + 8u * t));
+        // scale bytes of groups j = 4 (s & 3) + 2 u + (t >> 1), u = 0, 1: low nibbles
+        // at 96 + (j & 7), high bits at 104 + (j & 3)
+        const uint32_t j = 4 * (s & 3) + (t >> 1);
+        r.s0 = sb[off + 96 + (j & 7)] | (uint32_t)sb[off + 96 + ((j + 2) & 7)] << 8;
+        r.s1 = sb[off + 104 + (j & 3)] | (uint32_t)sb[off + 104 + ((j + 2) & 3)] << 8;
+        r.d = load_u16(sb + 108 + off);
+    } else {
+        const uint8_t* sb = base + (size_t)(s >> 2) * 84;
+        r.q = *reinterpret_cast<const u32x2_a2*>(sb + 16 + 32 * ((s & 3) >> 1) + (off + 8u * t));
+        r.s0 = *reinterpret_cast<const uint32_t*>(sb + 4 * (s & 3) + off);      // the stage's 4 groups
+        r.d = *reinterpret_cast<const uint32_t*>(sb + 80 + off);
+    }
+}
+
+// LDS of one K group's stage: x planes, w planes, floats per weight row (kScales
+// x BN), and for the types with mins the sums of x: 16 bytes per token and lane half.
+template <uint32_t T, int BM, int BN>
+struct Lay {
+    static constexpr int x = 0;
+    static constexpr int w = x + 3 * (BM / 32) * kTile;
+    static constexpr int sc = w + Traits<T>::kPlanes * (BN / 32) * kTile;
+    static constexpr int xs = (sc + 4 * Traits<T>::kScales * BN + 15) & ~15;
+    static constexpr int bytes = xs + (Traits<T>::kMin ? 32 * BM : 0);
+};
+
+template <uint32_t T, int BM, int BN>
+__device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, int s, int t, bool on) {
+    typedef Lay<T, BM, BN> L;
+    constexpr int PL = Traits<T>::kPlanes;
+    uint8_t* wt = st + L::w + (n >> 5) * kTile + (n & 31) * 16;
+    float* sc = reinterpret_cast<float*>(st + L::sc) + n;
+    if constexpr (T == T_BF16) {
+        *reinterpret_cast<u32x4*>(wt + t * kH) = on ? r.a : u32x4{0, 0, 0, 0};
+    } else if constexpr (T == T_F32 || T == T_F16) {
+#pragma unroll
+        for (int h = 0; h < (T == T_F32 ? 1 : 2); h++) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if constexpr (T == T_F32) v[i] = __uint_as_float(r.a[i]);
+                else v[i] = fp16_bits_to_f32(r.a[2 * h + (i >> 1)] >> (16 * (i & 1)));
+                v[i] = on ? v[i] : 0.0f;
+            }
+            u32x2 o[PL];
+            split4<PL>(v, o);
+            uint8_t* p = T == T_F32 ? wt + (t >> 1) * kH + 8 * (t & 1) : wt + t * kH + 8 * h;
+#pragma unroll
+            for (int k = 0; k < PL; k++) *reinterpret_cast<u32x2*>(p + k * (BN / 32) * kTile) = o[k];
+        }
+    } else {
+        // values 8t .. 8t + 7 of the stage's two 32-element groups 2j, 2j + 1
+        const int j = s & 3;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            float f = 1.0f;
+            if constexpr (T == T_Q3_K) {
+                const uint32_t k = 4 * j + 2 * u + (t >> 1);
+                const uint32_t lo = (r.s0 >> (8 * u)) & 0xffu, hb = (r.s1 >> (8 * u)) & 0xffu;
+                f = (float)((int)(((k < 8 ? lo : lo >> 4) & 15u) | (((hb >> (2 * (k >> 2))) & 3u) << 4)) - 32);
+            } else if constexpr (T == T_Q2_K) {
+                f = (float)((r.s0 >> (8 * (2 * u + (t >> 1)))) & 15u);
+            }
+            u32x4 o;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                uint32_t c;
+                if constexpr (T == T_Q5_K)
+                    c = ((r.q[i] >> (4 * u)) & 0x0f0f0f0fu) | (((r.h[i] >> (2 * j + u)) & 0x01010101u) << 4);
+                else
+                    c = (r.q[i] >> (4 * (j & 1) + 2 * u)) & 0x03030303u;
+                if constexpr (T == T_Q3_K) c |= ((r.h[i] >> (2 * j + u)) & 0x01010101u) << 2;      // code + 4
+                float v[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    v[k] = (float)((c >> (8 * k)) & 0xffu);
+                    if constexpr (T == T_Q3_K) v[k] = (v[k] - 4.0f) * f;
+                    if constexpr (T == T_Q2_K) v[k] *= f;
+                }
+                o[2 * i] = pk_bf16(v[0], v[1]);
+                o[2 * i + 1] = pk_bf16(v[2], v[3]);
+            }
+            *reinterpret_cast<u32x4*>(wt + (4 * u + t) * kH) = o;
+        }
+        if constexpr (T == T_Q5_K) {
+            if (t < 2) {
+                uint32_t s6, m6;
+                scale_min_k4(2 * j + t, r.hd.y, r.hd.z, r.hd.w, s6, m6);
+                sc[t * BN] = fp16_bits_to_f32(r.hd.x) * (float)s6;
+                sc[(2 + t) * BN] = (float)m6;
+            } else if (t == 2) {
+                sc[4 * BN] = fp16_bits_to_f32(r.hd.x >> 16);
+            }
+        } else if constexpr (T == T_Q2_K) {
+            sc[(2 + t) * BN] = (float)((r.s0 >> (8 * t + 4)) & 15u);
+            if (t < 2) sc[t * BN] = fp16_bits_to_f32(r.d >> (16 * t));
+        } else {
+            if (t == 0) sc[0] = fp16_bits_to_f32(r.d);
+        }
+    }
+}
+
+// One output in fp32. The pieces of an infinity are (inf, 0, 0) and its product
+// with a zero piece of a finite value is NaN, so are partial sums past the fp32
+// range with opposite signs, and the matrix unit takes pieces below 2^-126 as zero
+// (third pieces of values below 2^-108). Outputs that come out infinite, NaN or
+// nonzero and below 2^-80 (there by such values, not by cancellation: the 64-bit
+// sums of larger ones end in a whole zero or far above) are computed again so. A
+// NaN sum stays one.
+template <uint32_t T>
+__device__ __forceinline__ float plain_dot(const FactArgs& g, int m, int n) {
+    const float* x = g.x + (size_t)m * g.K;
+    const uint8_t* w = g.w + (size_t)n * g.rb;
+    float s = 0.0f, sm = 0.0f;            // the mins' sum apart, as the reference keeps it
+    for (int k = 0; k < g.K && s == s; k++) {
+        float mn = 0.0f;
+        if constexpr (T == T_Q2_K) {
+            const uint8_t* b = w + (k >> 8) * 84;
+            mn = fp16_bits_to_f32(rd16(b + 82)) * (float)(b[(k & 255) >> 4] >> 4);
+        } else if constexpr (T == T_Q5_K) {
+            const uint8_t* b = w + (k >> 8) * 176;
+            int sc, mi;
+            scale_min((k & 255) >> 5, b + 4, sc, mi);
+            mn = fp16_bits_to_f32(rd16(b + 2)) * (float)mi;
+        }
+        s = fmaf(x[k], dequant_one(T, w, k) + mn, s);
+        if constexpr (Traits<T>::kMin) sm = fmaf(x[k], mn, sm);
+    }
+    return s - sm;
+}
+__device__ __forceinline__ bool suspect(float v) {
+    const uint32_t e = (__float_as_uint(v) >> 23) & 0xffu;
+    return e == 255u || (e < 127u - 80u && v != 0.0f);
+}
+
+// MT x NT tiles of 32 x 32 per wave.
+template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
+__global__ void __launch_bounds__(64 * WM * WN * WK, 2)
+gemm_fact(FactArgs g) {
+    constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, GT = 64 * WM * WN;
+    typedef Lay<T, BM, BN> L;
+    typedef Traits<T> R;
+    constexpr int XPT = BM * 16 / GT, WPT = (BN * R::kTasks + GT - 1) / GT, PL = R::kPlanes;
+    static_assert(BM * 16 % GT == 0, "whole tasks");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x % GT, kg = WK > 1 ? (int)(threadIdx.x / GT) : 0;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % WM, wn = wave / WM;
+    // a group of one wave needs no barrier and one buffer: its LDS operations are in order
+    constexpr int NBUF = GT == 64 ? 1 : 2;
+    uint8_t* const lds = smem + kg * NBUF * L::bytes;
+
+    // tile order: as in the int8 product (one near-square block of tiles per XCD)
+    const int ntiles = g.ntm * g.ntn, bid = blockIdx.x;
+    const int q8 = ntiles >> 3, r8 = ntiles & 7, xcd = bid & 7;
+    const int tile = xcd * q8 + (xcd < r8 ? xcd : r8) + (bid >> 3);
+    constexpr int kGroup = 512 / BM;
+    const int grp = tile / (kGroup * g.ntn), in = tile - grp * kGroup * g.ntn;
+    const int gm = g.ntm - grp * kGroup < kGroup ? g.ntm - grp * kGroup : kGroup;
+    const int m0 = (grp * kGroup + in % gm) * BM, n0 = in / gm * BN;
+    const int nst = (g.K + 63) >> 6, iters = (nst + WK - 1) / WK;
+
+    float4 rx[XPT];
+    WReg<T> rw[WPT];
+    uint32_t xrow[XPT], woff[WPT];
+    const uint32_t quad = tid & 15;                 // 4-element piece of this thread's x tasks
+#pragma unroll
+    for (int i = 0; i < XPT; i++) {
+        const int row = (tid + i * GT) >> 4, m = m0 + row < g.M ? row : g.M - 1 - m0;
+        xrow[i] = (uint32_t)m * (uint32_t)g.K;
+    }
+#pragma unroll
+    for (int i = 0; i < WPT; i++) {
+        const int p = tid + i * GT, row = BN * R::kTasks % GT == 0 || p < BN * R::kTasks ? p / R::kTasks : 0;
+        const int n = n0 + row < g.N ? row : g.N - 1 - n0;
+        woff[i] = (uint32_t)n * (uint32_t)g.rb;
+    }
+    const float* const xbase = g.x + (size_t)m0 * g.K;
+    const uint8_t* const wbase = g.w + (size_t)n0 * g.rb;
+    // No load depends on a branch: pieces past K re-read the row's last elements (a
+    // stage past K the last stage's) and store() writes zeros for them.
+    auto load = [&](int s) {
+        s = s < nst ? s : nst - 1;
+        const uint32_t e = 64u * s + 4u * quad, ec = e < (uint32_t)g.K ? e : (uint32_t)g.K - 4u;
+#pragma unroll
+        for (int i = 0; i < XPT; i++) rx[i] = *reinterpret_cast<const float4*>(xbase + (xrow[i] + ec));
+#pragma unroll
+        for (int i = 0; i < WPT; i++)
+            w_load<T>(rw[i], wbase, woff[i], (uint32_t)g.rb, s, (tid + i * GT) % R::kTasks);
+    };
+    auto store = [&](int s, uint8_t* st) {
+        const bool on = 64 * s + 4 * (int)quad < g.K;
+#pragma unroll
+        for (int i = 0; i < XPT; i++) {
+            const int row = (tid + i * GT) >> 4;
+            const float v[4] = {on ? rx[i].x : 0.0f, on ? rx[i].y : 0.0f, on ? rx[i].z : 0.0f, on ? rx[i].w : 0.0f};
+            u32x2 o[3];
+            split4<3>(v, o);
+            uint8_t* p = st + L::x + (row >> 5) * kTile + (quad >> 1) * kH + (row & 31) * 16 + 8 * (quad & 1);
+#pragma unroll
+            for (int k = 0; k < 3; k++) *reinterpret_cast<u32x2*>(p + k * (BM / 32) * kTile) = o[k];
+            if constexpr (R::kMin) {
+                // sums of 16 (Q2_K) or 32 elements over 4 or 8 lanes, as three bf16
+                // pieces in K slots 0..2 and 4..6 of a lane half
+                float u = (v[0] + v[1]) + (v[2] + v[3]);
+                u = dpp_step<0xb1, 0xf>(u);
+                u = dpp_step<0x4e, 0xf>(u);
+                if constexpr (T == T_Q5_K) u = dpp_step<0x141, 0xf>(u);        // row_half_mirror
+                const float u1 = hi16(u), r = u - u1, u2 = hi16(r), u3 = r - u2;
+                const u32x2 rec = {__builtin_amdgcn_perm(__float_as_uint(u2), __float_as_uint(u1), 0x07060302u),
+                                   __float_as_uint(u3) >> 16};
+                u32x2* xs = reinterpret_cast<u32x2*>(st + L::xs) + 2 * ((quad >> 3) * BM + row);
+                if constexpr (T == T_Q2_K) {
+                    if ((quad & 3) == 0) xs[(quad >> 2) & 1] = rec;
+                } else {
+                    if ((quad & 3) == 0) xs[(quad >> 2) & 1] = quad & 4 ? u32x2{0, 0} : rec;
+                }
+            }
+        }
+        const int sw = s < nst ? s : nst - 1;
+#pragma unroll
+        for (int i = 0; i < WPT; i++) {
+            const int p = tid + i * GT, t = p % R::kTasks;
+            if (BN * R::kTasks % GT == 0 || p < BN * R::kTasks)
+                w_store<T, BM, BN>(rw[i], st, p / R::kTasks, sw, t, 64 * s + (R::kQuant ? 0 : 64 / R::kTasks * t) < g.K);
+        }
+    };
+
+    double sum[MT][NT][16];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < NT; r++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) sum[t][r][i] = 0.0;
+
+    const int col = lane & 31, half = lane >> 5;
+    auto compute = [&](const uint8_t* st) {
+        const uint8_t* xt = st + L::x + wm * MT * kTile + half * kH + col * 16;
+        const uint8_t* wt = st + L::w + wn * NT * kTile + half * kH + col * 16;
+        const float* sc = reinterpret_cast<const float*>(st + L::sc) + wn * NT * 32 + col;
+        f16v P[MT][NT];
+        float chain[T == T_Q5_K ? MT : 1][T == T_Q5_K ? NT : 1][16];
+        // Per unit (the stage; a 32-element block of Q5_K) the smaller products come
+        // first, so that only those of the first pieces are rounded at the sum's size.
+        constexpr int KU = T == T_Q5_K ? 2 : 4;
+        b8v B[KU][PL][NT];
+        auto frag_b = [&](int u, int k, int p) {
+#pragma unroll
+            for (int r = 0; r < NT; r++)
+                B[k][p][r] = *reinterpret_cast<const b8v*>(wt + (p * (BN / 32) + r) * kTile + 2 * (u * KU + k) * kH);
+        };
+#pragma unroll
+        for (int u = 0; u < 4 / KU; u++) {
+#pragma unroll
+            for (int k = 0; k < 2 * KU; k++) {
+                const int kk = k % KU;
+                b8v A[3][MT];
+                // with several planes of w the first is read again for its second use
+                if (k < KU) {
+#pragma unroll
+                    for (int p = 0; p < PL; p++) frag_b(u, kk, p);
+                } else if (PL > 1) {
+                    frag_b(u, kk, 0);
+                }
+#pragma unroll
+                for (int p = k < KU && PL == 1 ? 1 : 0; p < (k < KU ? 3 : 1); p++)
+#pragma unroll
+                    for (int t = 0; t < MT; t++)
+                        A[p][t] = *reinterpret_cast<const b8v*>(xt + (p * (BM / 32) + t) * kTile + 2 * (u * KU + kk) * kH);
+#pragma unroll
+                for (int r = 0; r < NT; r++)
+#pragma unroll
+                    for (int t = 0; t < MT; t++) {
+                        f16v c = k == 0 ? f16v{} : P[t][r];
+                        // pieces i of x and o - i of w, o = 2, 1, then 0
+                        if (k < KU) {
+#pragma unroll
+                            for (int o = 2; o >= 1; o--)
+#pragma unroll
+                                for (int i = 2; i >= 0; i--)
+                                    if (o - i >= 0 && o - i < PL)
+                                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i][t], B[kk][o - i][r], c, 0, 0, 0);
+                        } else {
+                            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0][t], B[kk][0][r], c, 0, 0, 0);
+                        }
+                        P[t][r] = c;
+                    }
+            }
+            if constexpr (T == T_Q5_K) {
+#pragma unroll
+                for (int r = 0; r < NT; r++) {
+                    const float ds = sc[u * BN + 32 * r];
+#pragma unroll
+                    for (int t = 0; t < MT; t++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++)
+                            chain[t][r][i] = u == 0 ? P[t][r][i] * ds : fmaf(P[t][r][i], ds, chain[t][r][i]);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < NT; r++) {
+            double d = 1.0, dm = 0.0;
+            b8v mb;
+            if constexpr (T == T_Q2_K || T == T_Q3_K) d = (double)sc[32 * r];
+            if constexpr (R::kMin) {
+                dm = -(double)sc[(T == T_Q5_K ? 4 : 1) * BN + 32 * r];
+                const float ma = T == T_Q5_K ? sc[(2 + half) * BN + 32 * r] : sc[(2 + 2 * half) * BN + 32 * r];
+                const float mc = T == T_Q5_K ? 0.0f : sc[(3 + 2 * half) * BN + 32 * r];
+                const uint32_t a1 = __float_as_uint(ma) >> 16, c1 = __float_as_uint(mc) >> 16;
+                const u32x4 o = {a1 | (a1 << 16), a1, c1 | (c1 << 16), c1};
+                mb = __builtin_bit_cast(b8v, o);
+            }
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                f16v am;
+                if constexpr (R::kMin) {
+                    const b8v xs = reinterpret_cast<const b8v*>(st + L::xs)[half * BM + (wm * MT + t) * 32 + col];
+                    am = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, mb, f16v{}, 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    float v;
+                    if constexpr (T == T_Q5_K) v = chain[t][r][i];
+                    else v = P[t][r][i];
+                    if constexpr (T == T_Q2_K || T == T_Q3_K) sum[t][r][i] = fma((double)v, d, sum[t][r][i]);
+                    else sum[t][r][i] += (double)v;
+                    if constexpr (R::kMin) sum[t][r][i] = fma((double)am[i], dm, sum[t][r][i]);
+                }
+            }
+        }
+    };
+
+    // Group kg takes the stages kg, kg + WK, ..; while one computes from one LDS
+    // buffer, the next is loaded into registers and then written to the other.
+    load(kg);
+    store(kg, lds);
+    __syncthreads();
+    for (int it = 0; it < iters; it++) {
+        const int next = (it + 1) * WK + kg;
+        if (WK > 1 && it == iters - 1) {        // few stages per group: no wait for a load nobody needs (19.6 -> 18.8 us)
+            compute(lds + (NBUF == 2 ? (it & 1) * L::bytes : 0));
+            break;
+        }
+        load(next);
+        compute(lds + (NBUF == 2 ? (it & 1) * L::bytes : 0));
+        if constexpr (NBUF == 1) __builtin_amdgcn_wave_barrier();
+        store(next, lds + (NBUF == 2 ? ((it + 1) & 1) * L::bytes : 0));
+        if constexpr (NBUF == 1) __builtin_amdgcn_wave_barrier();
+        else __syncthreads();
+    }
+
+    if constexpr (WK > 1) {
+        if constexpr (NBUF == 1) __syncthreads();      // every group is done with its buffer
+        // All groups leave their sums in LDS; group kg adds those of registers kg,
+        // kg + WK, .. in the groups' order (against one group adding the others' one
+        // after the other: BF16 N 4096 K 4096 M 12 21.4 -> 19.6 us).
+        double* red = reinterpret_cast<double*>(smem) + wave * MT * NT * 16 * 64 + lane;
+        constexpr int kGrp = WM * WN * MT * NT * 16 * 64;
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < NT; r++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) red[kg * kGrp + ((t * NT + r) * 16 + i) * 64] = sum[t][r][i];
+        __syncthreads();
+        for (int j = kg; j < MT * NT * 16; j += WK) {
+            double u = red[j * 64];
+#pragma unroll
+            for (int q = 1; q < WK; q++) u += red[q * kGrp + j * 64];
+            const int i = j & 15, n = n0 + (wn * NT + (j >> 4) % NT) * 32 + col;
+            const int m = m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+            if (m < g.M && n < g.N) {
+                const float v = (float)u;
+                g.y[(size_t)m * g.N + n] = suspect(v) ? plain_dot<T>(g, m, n) : v;
+            }
+        }
+        return;
+    }
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < NT; r++) {
+        const int n = n0 + (wn * NT + r) * 32 + col;
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int m = m0 + (wm * MT + t) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+                if (m < g.M && n < g.N) g.y[(size_t)m * g.N + n] = (float)sum[t][r][i];
+                bad |= suspect((float)sum[t][r][i]);
+            }
+    }
+    if (!__any(bad)) return;
+    for (int j = 0; j < MT * NT * 16; j++) {
+        const int i = j & 15, n = n0 + (wn * NT + (j >> 4) / MT) * 32 + col;
+        const int m = m0 + (wm * MT + (j >> 4) % MT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (m >= g.M || n >= g.N) continue;
+        float* y = g.y + (size_t)m * g.N + n;
+        if (suspect(*y)) *y = plain_dot<T>(g, m, n);
+    }
+}
+
+template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
+hipError_t launch_cfg(FactArgs g, hipStream_t st) {
+    constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
+    constexpr int red = WK > 1 ? WK * WM * WN * MT * NT * 8192 : 0;
+    constexpr int bufs = WK * (WM * WN == 1 ? 1 : 2) * Lay<T, BM, BN>::bytes;
+    constexpr int lds = bufs > red ? bufs : red;
+    static_assert(lds <= 160 * 1024, "LDS");
+    g.ntm = (g.M + BM - 1) / BM;
+    g.ntn = (g.N + BN - 1) / BN;
+    hipLaunchKernelGGL((gemm_fact<T, MT, NT, WM, WN, WK>), dim3((unsigned)(g.ntm * g.ntn)), dim3(64 * WM * WN * WK), lds,
+                       st, g);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+#ifdef LP_DEV
+int g_fact_cfg = -1;
+#endif
+
+namespace {
+// The tile forms (as the int8 product's; 64 x 128 where the planes of the weights
+// leave no LDS for 128 x 128). Measured, us, N 4096 K 4096:
+//   BF16  M 64   (256 tiles of 32 x 32)   32x32x8 24.8, 32x32x4 30, 64x64x2 49
+//         M 128  (512)                    32x32x4 41, 32x32x8 47, 64x64x2 51
+//         M 256  (256 tiles of 64 x 64)   64x64x2 54, 64x64 76, 32x32x4 77
+//         M 512  (512)                    64x64 95, 64x64x2 107, 128x128 123
+//         M 2048 (512 tiles of 128 x 128) 128x128 253, 64x64 343
+//   F32   M 128  32x32x6 85, 64x64 119      M 256  64x64 119, 64x128 165
+//         M 512  64x128 169, 64x64 225
+enum Form { F32X32X8, F32X32X4, F64X64X2, F64X64, F64X128, F128X128 };
+
+template <uint32_t T>
+Form pick_form(int M, int N) {
+#ifdef LP_DEV
+    if (g_fact_cfg >= 0) return (Form)g_fact_cfg;
+#endif
+    const long cus = device_cu_count();
+    auto tiles = [&](int b) { return (long)((M + b - 1) / b) * ((N + b - 1) / b); };
+    constexpr bool one = Traits<T>::kPlanes == 1;
+    if (tiles(32) <= cus) return F32X32X8;
+    if (tiles(32) <= 2 * cus || M <= 32) return one ? F32X32X4 : F32X32X8;
+    if (tiles(64) <= cus) return one ? F64X64X2 : F64X64;
+    if (!one) return F64X128;
+    const long r64 = (tiles(64) + 2 * cus - 1) / (2 * cus), r128 = (tiles(128) + cus - 1) / cus;
+    return 1.4 * r128 < r64 ? F128X128 : F64X64;
+}
+
+template <uint32_t T>
+hipError_t launch_t(const FactArgs& g, hipStream_t st) {
+    constexpr bool one = Traits<T>::kPlanes == 1;
+    switch (pick_form<T>(g.M, g.N)) {
+        case F32X32X8: return launch_cfg<T, 1, 1, 1, 1, one ? 8 : 6>(g, st);
+        case F32X32X4: return launch_cfg<T, 1, 1, 1, 1, one ? 4 : 6>(g, st);
+        case F64X64X2: return launch_cfg<T, 1, 1, 2, 2, one ? 2 : 1>(g, st);
+        case F64X64: return launch_cfg<T, 1, 1, 2, 2, 1>(g, st);
+        case F64X128: if constexpr (!one) return launch_cfg<T, 1, 2, 2, 2, 1>(g, st); [[fallthrough]];
+        default: return launch_cfg<T, 1, 2, one ? 4 : 2, 2, 1>(g, st);
+    }
+}
+}  // namespace
+
+// Where this product beats the GEMVs, which read the weights once per 4 rows: up to
+// 32 rows its time depends on K alone (one round of tiles), theirs on M N K, so the
+// line is a number of outputs, for F16 and F32 one per round of tiles; twice as many at K <= 2048, where its launch and last
+// reduction weigh more. Measured (us, GEMV against this): K 4096: BF16 N 4096 M 5
+// 18.7 / 19, M 6 21.0 / 19.5, M 12 31.5 / 18.8, M 33 82.5 / 20.0; N 1024 M 12 9.2 /
+// 19, M 33 23.4 / 18.3; Q5_K N 4096 M 6 30.4 / 27.7, M 12 66 / 28; Q3_K M 6 29.1 /
+// 26.9; Q2_K M 6 22.3 / 26, M 8 28.9 / 26.9; F16, F32 (more products) N 4096 M 8
+// 24.4, 28.7 / 32, 37, M 12 37.4, 40.5 / 32.1, 36.5; N 14336 (two rounds of tiles) F16
+// M 6 65.8 / 62.8, F32 M 6 86 / 73, N 8200 F16 M 8 52.5 / 61. K 1024, N 4096: BF16 M 8 7.9 / 7.2, M 12 10.5 / 7.2; F16 M 12 11.2 / 11.5,
+// M 33 27 / 11.5. Large: N 14336 K 4096 M 200 BF16 1690 -> 140, Q5_K 2660 -> 186, Q3_K
+// 2018 -> 150, Q2_K 1556 -> 168, F16 1547 -> 280, F32 2057 -> 329.
+bool fact_gemm_preferred(uint32_t type, int M, int K, int N) {
+    const long cus = device_cu_count(), rounds = ((long)((M + 31) / 32) * ((N + 31) / 32) + cus - 1) / cus;
+    const bool many = type == T_F32 || type == T_F16;
+    const long line = many ? 12000 + 37000 * rounds : type == T_Q2_K ? 32000 : 24000;
+    return M >= (type == T_F16 ? 6 : 5) && (long)M * N >= (K <= 2048 ? 2 * line : line);
+}
+
+hipError_t launch_gemm_fact(uint32_t type, const uint8_t* w, const float* x, float* y, int M, int K, int N,
+                            hipStream_t st) {
+    if (M <= 0 || N <= 0) return hipSuccess;
+    const FactArgs g{w, x, y, M, N, K, fact_row_bytes(type, K), 0, 0};
+    switch (type) {
+        case T_F32: return launch_t<T_F32>(g, st);
+        case T_F16: return launch_t<T_F16>(g, st);
+        case T_BF16: return launch_t<T_BF16>(g, st);
+        case T_Q2_K: return launch_t<T_Q2_K>(g, st);
+        case T_Q3_K: return launch_t<T_Q3_K>(g, st);
+        case T_Q5_K: return launch_t<T_Q5_K>(g, st);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace lp
+
+#ifdef LP_DEV
+extern "C" int lp_dev_fact(int cfg, const float* x, const uint8_t* w, uint32_t type, float* y, int M, int K, int N,
+                           unsigned long rb, void* stream) {
+    lp::g_fact_cfg = cfg;
+    return (int)lp::launch_gemm_fact(type, w, x, y, M, K, N, (hipStream_t)stream);
+}
+#endif

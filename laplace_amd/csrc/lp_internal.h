@@ -61,6 +61,12 @@ size_t fact_row_bytes(uint32_t type, int K);
 hipError_t launch_gemv_fact(uint32_t type, const uint8_t* w, const float* x, float* y, int M, int K, int N,
                             hipStream_t st);
 
+// Tiled bf16-MFMA product at fp32 precision for the same types (lp_gemm_fact.hip);
+// launch_gemv_fact takes it where fact_gemm_preferred says so.
+bool fact_gemm_preferred(uint32_t type, int M, int K, int N);
+hipError_t launch_gemm_fact(uint32_t type, const uint8_t* w, const float* x, float* y, int M, int K, int N,
+                            hipStream_t st);
+
 hipError_t launch_quantize(const float* x, int M, int K, const ActView& A, hipStream_t st);
 hipError_t launch_gemv(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K,
                        int N, hipStream_t st);

@@ -1,0 +1,152 @@
+"""The tiled bf16-MFMA product (F32, F16, BF16, Q2_K, Q3_K, Q5_K prompt rows) at the
+edges of its tiles and forms, against 64-bit products and the oracle."""
+import numpy as np
+import pytest
+
+from hip_util import normwise
+from test_gpu_fact import BF16, F16, F32, FACT, Q2_K, Q3_K, Q5_K, fact_weights, gemm_dev
+
+pytestmark = pytest.mark.gpu
+DENSE = {"F32": F32, "F16": F16, "BF16": BF16}
+
+# Per 64 elements (32 of Q5_K) the leading products are summed in fp32: at most 64
+# half-ulps of a partial sum, 64 * 2^-25 = 2e-6; the dropped products and the result's
+# rounding are below 2^-22. The oracle rounds an fp32 sum K <= 2048 times: with random
+# signs ~sqrt(2048) half-ulps, 1.4e-6.
+TOL = 4e-6
+
+# (M, N, K): one token and one row past a 32- and 64-tile, K ending 32 elements into
+# a 64-element stage (the unquantized types), fewer stages than K groups
+SHAPES = [(33, 3001, 256), (65, 1537, 512), (8, 12289, 768), (127, 449, 2048)]
+TAILS = [(33, 3001, 32), (65, 1537, 96), (8, 12289, 288), (127, 801, 1056)]
+# M and N that take each form: 32x32 with 8 (6) and 4 K groups, 64x64 with 2 and 1,
+# 64x128, 128x128 (and its edges)
+FORMS = [(31, 8200, 256), (40, 8200, 256), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256)]
+CASES = [(t, *s) for t in FACT for s in SHAPES + FORMS] + [(t, *s) for t in DENSE for s in TAILS]
+
+
+@pytest.mark.parametrize("name,M,N,K", CASES)
+def test_fact_gemm_matches_oracle(orc, name, M, N, K):
+    print(f"fact gemm {name} M={M} N={N} K={K}", flush=True)
+    t = FACT[name]
+    w = fact_weights(t, K, N, seed=M + N + K + t)
+    x = np.random.default_rng(M + 1).standard_normal((M, K)).astype(np.float32)
+    x[M // 2, :32] = 0.0
+    y = gemm_dev(t, x, w, N)
+    rows = np.unique(np.linspace(0, N - 1, 48).astype(int))     # both ends and between
+    rb = len(w) // N
+    sub = np.concatenate([w[r * rb:(r + 1) * rb] for r in rows])
+    assert normwise(y[:, rows], orc.gemm_scalar(t, x, sub, len(rows))) <= TOL
+
+
+def dense(t, v):
+    if t == F16:
+        return v.astype(np.float16).astype(np.float32), v.astype(np.float16).view(np.uint8).reshape(-1)
+    if t == BF16:
+        u = v.view(np.uint32) & 0xffff0000
+        return u.view(np.float32), (u >> 16).astype(np.uint16).view(np.uint8).reshape(-1)
+    return v, v.view(np.uint8).reshape(-1)
+
+
+@pytest.mark.parametrize("scale", [1e-35, 1.0, 1e30])
+@pytest.mark.parametrize("name", list(DENSE))
+def test_fact_gemm_pieces_keep_fp32(name, scale):
+    """Every value is multiplied with its 24 bits, at any size: one product per
+    output leaves its own rounding and the pieces' last bits."""
+    t = DENSE[name]
+    M, N, K = 64, 1600, 64
+    rng = np.random.default_rng(3)
+    x = np.zeros((M, K), np.float32)
+    x[np.arange(M), np.arange(M)] = ((0.5 + rng.random(M)) * scale).astype(np.float32)
+    v, wb = dense(t, rng.standard_normal((N, K)).astype(np.float32))
+    y = gemm_dev(t, x, wb, N)
+    ref = x.astype(np.float64) @ v.astype(np.float64).T
+    assert np.all(np.abs(y - ref) <= 4 * 2.0 ** -24 * np.abs(ref) + 2.0 ** -149)
+
+
+@pytest.mark.parametrize("name", ["Q2_K", "Q3_K", "Q5_K"])
+def test_fact_gemm_quantized_extremes(orc, name):
+    """Rows with an infinity, a NaN, values as large and as small as the codes leave room for
+    match the oracle; the rows beside them stay as they are."""
+    t = FACT[name]
+    M, N, K = 40, 1700, 512
+    w = fact_weights(t, K, N, seed=4)
+    x = np.random.default_rng(6).standard_normal((M, K)).astype(np.float32)
+    x[1, 7], x[2, 500], x[M - 1, 511] = np.inf, np.nan, -np.inf
+    x[3, 9] = 1e36
+    x[4] *= 1e-36
+    y = gemm_dev(t, x, w, N)
+    with np.errstate(all="ignore"):
+        ref = orc.gemm_scalar(t, x, w, N)
+    assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
+    for m in range(M):
+        f = np.isfinite(ref[m])
+        assert np.array_equal(y[m][~f & ~np.isnan(ref[m])], ref[m][~f & ~np.isnan(ref[m])])
+        if f.any():
+            s = np.abs(ref[m][f]).max()
+            assert normwise(y[m][f] / s, ref[m][f] / s) <= TOL, m
+
+
+@pytest.mark.parametrize("M,N", [(40, 2500), (70, 8200), (200, 24600)])
+@pytest.mark.parametrize("name", list(DENSE))
+def test_fact_gemm_non_finite(name, M, N):
+    """Infinities and NaN on either side, and sums past the fp32 range, come out as
+    the plain products give them; all other outputs stay exact."""
+    t = DENSE[name]
+    K = 96
+    rng = np.random.default_rng(5)
+    x = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    v = rng.integers(-4, 5, (N, K)).astype(np.float32)
+    x[x == 0] = 1
+    v[v == 0] = 1
+    x[1, 3], x[2, 90], x[M - 1, 95], x[M - 2, 5] = np.inf, -np.inf, np.nan, np.inf
+    v[4, 7], v[N - 1, 0], v[N // 2, 9] = np.inf, -np.inf, np.nan
+    x[3, 10], x[4, 10] = 3.4028235e38, -3.38e38
+    v, wb = dense(t, v)
+    with np.errstate(all="ignore"):
+        ref = (x.astype(np.float64)[:, None, :] * v.astype(np.float64)[None, :64]).sum(-1)
+        last = (x.astype(np.float64)[:, None, :] * v.astype(np.float64)[None, -64:]).sum(-1)
+        mid = (x.astype(np.float64) * v.astype(np.float64)[N // 2]).sum(-1)
+    y = gemm_dev(t, x, wb, N)
+    for got, want in ((y[:, :64], ref), (y[:, -64:], last), (y[:, N // 2], mid)):
+        with np.errstate(all="ignore"):
+            want = want.astype(np.float32)
+        # a large value beside small ones: those of the sum are lost in either order
+        near = np.isclose(got, want, rtol=2.0 ** -22, atol=0, equal_nan=True)
+        assert near.all(), np.argwhere(~near)[:5]
+
+
+@pytest.mark.parametrize("name", ["F16", "BF16"])
+def test_fact_gemm_unaligned_weights(name):
+    """2-byte aligned weights give the aligned call's bits."""
+    import torch
+    from hip_util import L, stream, to_dev
+    t = FACT[name]
+    M, N, K = 40, 2500, 96
+    w = fact_weights(t, K, N, seed=1)
+    x = np.random.default_rng(2).standard_normal((M, K)).astype(np.float32)
+    want = gemm_dev(t, x, w, N)
+    for off in (2, 6):
+        buf = to_dev(np.concatenate([np.zeros(off, np.uint8), w]))
+        y = torch.empty(M * N, dtype=torch.float32, device="cuda")
+        xd = to_dev(x)
+        assert L().lp_gemm_dev(xd.data_ptr(), buf.data_ptr() + off, t, y.data_ptr(), M, K, N, None, 0, stream()) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy().reshape(M, N).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("name", list(FACT))
+def test_fact_gemm_line(name):
+    """On either side of the line between the GEMVs and this product (24000 outputs,
+    32000 of Q2_K, 49000 in one round of tiles of F16 and F32, twice that up to K = 2048;
+    5 rows, 6 of F16) the rows agree."""
+    t = FACT[name]
+    line = 49000 if t in (F32, F16) else 32000 if t == Q2_K else 24000
+    m0 = 6 if t == F16 else 5
+    rng = np.random.default_rng(8)
+    for M, N, K in ((m0, -(-line // m0), 4096), (16, -(-line // 16), 4096), (16, -(-line // 8), 512)):
+        w = fact_weights(t, K, N, seed=N)
+        x = rng.standard_normal((M, K)).astype(np.float32)
+        y = gemm_dev(t, x, w, N)
+        for part in (gemm_dev(t, x[:m0 - 1], w, N), gemm_dev(t, x[:2], w, N)):
+            assert normwise(y[:len(part)], part) <= TOL
