@@ -488,7 +488,7 @@ gemm_fact(FactArgs g) {
     }
 
     if constexpr (WK > 1) {
-        if constexpr (NBUF == 1) __syncthreads();      // every group is done with its buffer
+        __syncthreads();      // every wave is done with its buffer
         // All groups leave their sums in LDS; group kg adds those of registers kg,
         // kg + WK, .. in the groups' order (against one group adding the others' one
         // after the other: BF16 N 4096 K 4096 M 12 21.4 -> 19.6 us).

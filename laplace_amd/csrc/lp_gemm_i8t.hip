@@ -568,7 +568,7 @@ gemm_i8t(I8tArgs g) {
         flush();
     }
     if constexpr (WK > 1) {
-        if constexpr (NBUF == 1) __syncthreads();      // every group is done with its buffer
+        __syncthreads();      // every wave is done with its buffer
         // All groups leave their sums in LDS; group kg adds those of registers kg,
         // kg + WK, .. in the groups' order (against one group adding the others' one
         // after the other: Q8_0 N 4096 K 4096 M 16 13.1 -> 11.6 us with the quantizer).
