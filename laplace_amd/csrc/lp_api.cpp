@@ -434,12 +434,14 @@ static int check_moe(uint32_t type, const void* w, int T, int topk, int E, int K
     return LP_OK;
 }
 
-// Pairs per routed group below the 16-pair MFMA groups: 8 on the row-quad
+// Pairs per routed group: 32 and more on the tiled int8 product where experts have
+// enough of them (moe_i8t_group), else 8 on the row-quad
 // kernel once experts average more than 2 pairs (groups of 4 would split
 // many experts into groups that each read the expert again; measured at 128
 // experts, 64 tokens, top-8: 133 vs 147 us), else 4 on the GEMV kernels
 // (one or two pairs per expert: 39 vs 41 us at one token, 52 vs 58 at four).
-static int moe_group_size(uint32_t type, int K, int P, int E) {
+static int moe_group_size(uint32_t type, int rows, int K, int P, int E) {
+    if (const int gs = moe_i8t_group(type, rows, K, P, E)) return gs;
     return rq_moe_supported(type, K) && P > 2 * E ? kRqMoeGroup : 4;
 }
 
@@ -450,13 +452,7 @@ static int moe_q(const float* x, int multi, const int* idx, const uint8_t* w, ui
     const int P = T * topk, rows = multi ? P : T;
     const ActView A = ws_view(ws, rows, K);
     void* route = static_cast<uint8_t*>(ws) + act_bytes(rows, K);
-    // groups of <= 16 pairs on the int8 MFMA kernel pay off when experts are
-    // chosen by more than 8 pairs on average (prefill; at 128 experts, top-8:
-    // 10 per expert 259 vs 274 us on the GEMV kernels, 8 per expert 246 vs
-    // 236 us; 6 per expert 177 vs 137 us); decode-sized batches stay on the
-    // GEMV kernels
-    const bool mf = moe_mf_supported(type, K) && P > 8 * E;
-    const int gs = mf ? 16 : moe_group_size(type, K, P, E);
+    const int gs = moe_group_size(type, rows, K, P, E);
     if (kMoeFuseQuantRoute) {
         // one launch for the quantization and the route table (the route
         // kernel alone is one short workgroup)
@@ -868,12 +864,9 @@ int lp_moe_ffn_dev(const float* x, int T, int H, const uint8_t* router_w, uint32
     int* idx = topk_idx ? topk_idx : f.idx;
     float* wts = topk_w ? topk_w : f.wts;
     const int P = T * top_k;
-    // Decode-sized batches (neither expert pass on the MFMA kernel): the norm
-    // and GeGLU kernels also write the int8 blocks the expert GEMVs read, and
-    // one route table serves both passes.
-    const bool fused = !(moe_mf_supported(gate_up_type, H) && P > 8 * n_exp) &&
-                       !(moe_mf_supported(down_type, inter) && P > 8 * n_exp) && H % 32 == 0 &&
-                       inter % 32 == 0 && reinterpret_cast<uintptr_t>(router_scale) % 16 == 0 &&
+    // The norm and GeGLU kernels also write the int8 blocks the expert products
+    // read, and one route table serves both passes.
+    const bool fused = H % 32 == 0 && inter % 32 == 0 && reinterpret_cast<uintptr_t>(router_scale) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(pre_norm) % 16 == 0;
     if (fused && moe_norm_router_supported(T, H, router_type, router_w, router_scale, pre_norm)) {
         // few tokens: one launch for the norms and the router (measured at
@@ -888,9 +881,10 @@ int lp_moe_ffn_dev(const float* x, int T, int H, const uint8_t* router_w, uint32
             return rc;
     }
     if (fused) {
-        // one route table for both products: groups of 8 only if both run on
-        // the row-quad kernel; for a few tokens the top-k kernel builds it
-        const int gs = std::min(moe_group_size(gate_up_type, H, P, n_exp), moe_group_size(down_type, inter, P, n_exp));
+        // one route table for both products: the smaller of two tiled groups; groups
+        // of 8 only if both run on the row-quad kernel
+        const int g0 = moe_group_size(gate_up_type, T, H, P, n_exp), g1 = moe_group_size(down_type, P, inter, P, n_exp);
+        const int gs = g0 == g1 || (g0 >= 32 && g1 >= 32) ? std::min(g0, g1) : 4;
         if (moe_topk_route_supported(T)) {
             LP_HIP(launch_moe_topk_route(f.logits, T, n_exp, top_k, idx, wts, f.route, gs, st));
         } else {

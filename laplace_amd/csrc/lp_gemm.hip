@@ -744,8 +744,6 @@ quant_planes_kernel(const float* __restrict__ x, int K, Planes P, float* __restr
 
 constexpr int kMfWaves = 8;
 constexpr int kMfTiles = 2;         // 16-row tiles per workgroup (every wave takes all of them)
-constexpr int kMfMoeWaves = 2;      // grouped MoE: waves per workgroup
-constexpr int kMfMoeRows = 64;    // grouped MoE: weight rows per workgroup (at least two sets)
 constexpr int kMfMaxM = 16;
 // Measured on MI355X (Q4_K 18944 x 3584): the GEMV tile kernel is faster
 // up to M = 4, the small-M MFMA kernels from M = 5 to 16.
@@ -874,69 +872,27 @@ gemv_q4k_mf(MfArgs a) {
 // 4*(lane/16)+r, column = lane%16.
 typedef int i4v __attribute__((ext_vector_type(4)));
 
-// K-slices for a row of nsb super-blocks over nwv waves: the largest power
-// of two <= min(nsb, nwv) (nwv a power of two)
-__host__ __device__ inline int mf_kslices(int nsb, int nwv) {
-    int k = 1;
-    while (2 * k <= nsb && 2 * k <= nwv) k *= 2;
-    return k;
-}
-
-// MOE: blockIdx.y is a routed group (expert, first pair, n <= 16 pairs): the
-// group's activation rows (token, or pair in the multi form) and outputs
-// (pair rows) replace rows 0..M-1.
-// TL 16-row tiles per row set, NWV waves (K-slices); ri row sets per
-// workgroup, one after another, all served by one activation staging. RWS:
-// as many K-slices as the row has super-blocks (a power of two, at most
-// NWV), the remaining waves on further row tiles of the set.
-template <bool MOE, int TL = kMfTiles, int NWV = kMfWaves, bool RWS = false>
+// TL 16-row tiles per workgroup, NWV waves (K-slices).
+template <int TL = kMfTiles, int NWV = kMfWaves>
 __global__ void __launch_bounds__(64 * NWV)
-gemv_q4k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restrict__ y, int M, int K, int N,
-              const uint8_t* __restrict__ route, int max_groups, int multi, int topk, long ebytes, int ri = 1) {
+gemv_q4k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restrict__ y, int M, int K, int N) {
     __shared__ f4v red[NWV][TL][64];
     extern __shared__ __attribute__((aligned(16))) float sdx[];   // [nb][16] xd, then [nb][16] xs
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int tok = lane & 15, g = lane >> 4;
     const int nsb = K >> 8, nb = K >> 5;
-    const int* pairs = nullptr;
-    int first = 0;
-    if constexpr (MOE) {
-        if ((int)blockIdx.y >= *reinterpret_cast<const int*>(route)) return;
-        const int4 gd = reinterpret_cast<const int4*>(route + 16)[blockIdx.y];
-        pairs = reinterpret_cast<const int*>(route + 16 + (size_t)max_groups * 16);
-        first = gd.y;
-        M = gd.z;
-        w += (size_t)gd.x * ebytes;
-    }
-    auto act_row = [&](int t) -> int {
-        if constexpr (MOE) {
-            const int p = pairs[first + t];
-            return multi ? p : p / topk;
-        } else {
-            return t;
-        }
-    };
     float* sxs = sdx + (size_t)nb * 16;
     for (int i = threadIdx.x; i < nb * 16; i += blockDim.x) {
         const int b = i >> 4, t = i & 15;
-        const size_t r = t < M ? (size_t)act_row(t) : 0;
-        sdx[i] = t < M ? A.d[r * nb + b] : 0.0f;
-        sxs[i] = t < M ? A.sum[r * nb + b] : 0.0f;
+        sdx[i] = t < M ? A.d[(size_t)t * nb + b] : 0.0f;
+        sxs[i] = t < M ? A.sum[(size_t)t * nb + b] : 0.0f;
     }
     __syncthreads();
     const bool tv = tok < M;
-    const int8_t* aq = A.qs + (size_t)act_row(tv ? tok : 0) * K + 8 * g;
-    // RWS: K-slices of whole super-blocks, as many as the row has (a power of
-    // two, at most NWV), the other waves on further row tiles
-    const int ks_n = RWS ? mf_kslices(nsb, NWV) : NWV, rw_n = NWV / ks_n;
-    const int ks = wv % ks_n, rw = wv / ks_n;
-    const int sb0 = ks * nsb / ks_n, sb1 = (ks + 1) * nsb / ks_n;
-    // ri consecutive row sets per workgroup: the activation staging above
-    // serves all of them
-    for (int it = 0; it < ri; it++) {
-    const int rbase = (blockIdx.x * ri + it) * rw_n * (16 * TL);
-    if (rbase >= N) break;
-    const int row0 = rbase + rw * (16 * TL) + (lane & 15);
+    const int8_t* aq = A.qs + (size_t)(tv ? tok : 0) * K + 8 * g;
+    const int sb0 = wv * nsb / NWV, sb1 = (wv + 1) * nsb / NWV;
+    const int rbase = blockIdx.x * (16 * TL);
+    const int row0 = rbase + (lane & 15);
     const uint8_t* wr[TL];
 #pragma unroll
     for (int t = 0; t < TL; t++) {
@@ -998,25 +954,15 @@ gemv_q4k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restri
     for (int t = 0; t < TL; t++) red[wv][t][lane] = acc[t];
     __syncthreads();
     // each output tile summed over its K-slices in a fixed order
-    for (int o = wv; o < rw_n * TL; o += NWV) {
-        const int ro = o / TL, t = o % TL;
-        f4v sum = red[ro * ks_n][t][lane];
-        for (int i = 1; i < ks_n; i++) sum += red[ro * ks_n + i][t][lane];
-        const int row = rbase + ro * (16 * TL) + 16 * t + (lane & 15);
+    for (int t = wv; t < TL; t += NWV) {
+        f4v sum = red[0][t][lane];
+        for (int i = 1; i < NWV; i++) sum += red[i][t][lane];
+        const int row = rbase + 16 * t + (lane & 15);
         if (row < N) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int tt = 4 * g + r;
-                if (tt < M) {
-                    int yr;
-                    if constexpr (MOE) yr = pairs[first + tt];
-                    else yr = tt;
-                    y[(size_t)yr * N + row] = sum[r];
-                }
-            }
+            for (int r = 0; r < 4; r++)
+                if (4 * g + r < M) y[(size_t)(4 * g + r) * N + row] = sum[r];
         }
-    }
-    if (ri > 1) __syncthreads();                  // red is reused by the next row set
     }
 }
 
@@ -1195,11 +1141,10 @@ hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, f
         // of K 14336): 16-row workgroups of 16 waves (M=16 42.6 -> 34.1 us
         // there; at 14336 x 4096 the 32-row form is faster, 26.3 vs 36.7)
         if ((N + 31) / 32 < device_cu_count())
-            hipLaunchKernelGGL((gemv_q4k_i8mf<false, 1, 16>), dim3((N + 15) / 16), dim3(1024), shm, st, w, rbq, A, y,
-                               M, K, N, nullptr, 0, 0, 1, 0L);
+            hipLaunchKernelGGL((gemv_q4k_i8mf<1, 16>), dim3((N + 15) / 16), dim3(1024), shm, st, w, rbq, A, y,
+                               M, K, N);
         else
-            hipLaunchKernelGGL(gemv_q4k_i8mf<false>, grid, dim3(64 * kMfWaves), shm, st, w, rbq, A, y, M, K, N,
-                               nullptr, 0, 0, 1, 0L);
+            hipLaunchKernelGGL(gemv_q4k_i8mf<>, grid, dim3(64 * kMfWaves), shm, st, w, rbq, A, y, M, K, N);
     }
     return hipGetLastError();
 }
@@ -1355,33 +1300,6 @@ hipError_t launch_gemm(uint32_t type, const uint8_t* w, const ActView& A, void* 
                                               : launch_planes_from_act(A, planes, M, K, st, N, y);
     if (e != hipSuccess) return e;
     return launch_gemm_planes(type, w, planes, y, M, K, N, st, true);
-}
-
-bool moe_mf_supported(uint32_t type, int K) {
-    return type == T_Q4_K && K % 256 == 0 && (size_t)(K / 32) * 16 * 8 <= 64 * 1024;
-}
-
-hipError_t launch_moe_i8mf(const uint8_t* w, const ActView& A, const void* route, int max_groups, int multi,
-                           int topk, float* y, int K, int N, hipStream_t st) {
-    if ((size_t)(K / 32) * 16 * 8 > 64 * 1024) return hipErrorInvalidValue;
-    const long rb = (long)row_bytes(T_Q4_K, K);
-    // two waves (two K-slices) per workgroup, row sets of rw rows, ri of them
-    // per workgroup: kMfMoeRows rows, at least two sets. Measured at 128
-    // experts, top-8, 160 / 256 / 512 tokens (us per layer): 8 waves with one
-    // 32-row set and 8 K-slices for every K - / 358 / 591, 4 sets 313 / 496
-    // (256 / 512), with fewer K-slices at short K 291 / 451, two sets at K 768
-    // 219 / 281 / 444; 512 rows per workgroup 382 / 455 (too few
-    // workgroups); then 4 waves 194-198 / 254-258 / 408-410, 2 waves with 64
-    // rows 195-198 / 253 / 394-398 (32 rows: the same; 128: 271-273 at 256
-    // tokens), 1 wave 193-197 / 274-277 / 404-407, 16 waves 287 / 472
-    constexpr int NWM = kMfMoeWaves;
-    const int rw = 16 * kMfTiles * (NWM / mf_kslices(K / 256, NWM));
-    const int ri = rw < kMfMoeRows ? kMfMoeRows / rw : 2;
-    const int rows = rw * ri;
-    hipLaunchKernelGGL((gemv_q4k_i8mf<true, kMfTiles, NWM, true>), dim3((N + rows - 1) / rows, max_groups),
-                       dim3(64 * NWM), (size_t)(K / 32) * 16 * 8, st, w, rb, A, y, 0, K, N,
-                       static_cast<const uint8_t*>(route), max_groups, multi, topk, rb * N, ri);
-    return hipGetLastError();
 }
 
 }  // namespace lp

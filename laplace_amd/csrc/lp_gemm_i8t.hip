@@ -75,6 +75,11 @@ struct I8tArgs {
     int M, N, K;
     size_t rb;
     int ntm, ntn;
+    // grouped MoE rows: the route table (lp_route.h), its pairs' offset, bytes of one
+    // expert's weights
+    const uint8_t* route;
+    int mg, multi, topk;
+    long ebytes;
 };
 
 // Per-type staging of one 128-element stage of BN weight rows by GT threads.
@@ -292,8 +297,9 @@ __device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, in
     }
 }
 
-// MT x NT tiles of 32 x 32 per wave.
-template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
+// MT x NT tiles of 32 x 32 per wave. MOE: a token tile is a routed group (expert,
+// first pair, n <= BM pairs); its rows are gathered and scattered by pair.
+template <uint32_t T, int MT, int NT, int WM, int WN, int WK, bool MOE>
 __global__ void __launch_bounds__(64 * WM * WN * WK, 2)
 gemm_i8t(I8tArgs g) {
     constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, GT = 64 * WM * WN;
@@ -313,13 +319,33 @@ gemm_i8t(I8tArgs g) {
     // turn), ordered in groups of kGroup token tiles that walk the weight tiles
     // together: the tiles in flight on an XCD then form a near-square block, whose
     // operands its L2 serves
-    const int ntiles = g.ntm * g.ntn, bid = blockIdx.x;
+    const int bid = blockIdx.x;
+    if constexpr (MOE) {
+        g.ntm = *reinterpret_cast<const int*>(g.route);
+        if (bid >= g.ntm * g.ntn) return;
+    }
+    const int ntiles = g.ntm * g.ntn;
     const int q8 = ntiles >> 3, r8 = ntiles & 7, xcd = bid & 7;
     const int tile = xcd * q8 + (xcd < r8 ? xcd : r8) + (bid >> 3);
-    constexpr int kGroup = 512 / BM;
+    constexpr int kGroup = MOE ? 1 : 512 / BM;
     const int grp = tile / (kGroup * g.ntn), in = tile - grp * kGroup * g.ntn;
     const int gm = g.ntm - grp * kGroup < kGroup ? g.ntm - grp * kGroup : kGroup;
-    const int m0 = (grp * kGroup + in % gm) * BM, n0 = in / gm * BN;
+    int m0 = (grp * kGroup + in % gm) * BM;
+    const int n0 = in / gm * BN;
+    const int* pairs = nullptr;
+    if constexpr (MOE) {
+        const int4 gd = reinterpret_cast<const int4*>(g.route + 16)[grp];
+        pairs = reinterpret_cast<const int*>(g.route + 16 + (size_t)g.mg * 16) + gd.y;
+        g.w += gd.x * g.ebytes;
+        g.M = gd.z;
+        m0 = 0;
+    }
+    auto arow = [&](int m) {                     // the activation row of a token
+        if constexpr (!MOE) return m;
+        const int p = pairs[m];
+        return g.multi ? p : p / g.topk;
+    };
+    auto yrow = [&](int m) { return (size_t)(MOE ? pairs[m] : m) * g.N; };
     const int nb = g.K >> 5;
     const int nst = (nb + 3) >> 2, iters = (nst + 2 * WK - 1) / (2 * WK);
 
@@ -330,13 +356,13 @@ gemm_i8t(I8tArgs g) {
 #pragma unroll
     for (int i = 0; i < APT; i++) {
         const int p = tid + i * GT, m = m0 + (p >> 3) < g.M ? p >> 3 : g.M - 1 - m0;
-        aoff[i] = (uint32_t)m * (uint32_t)g.K + 16u * (p & 7);
+        aoff[i] = (uint32_t)arow(m) * (uint32_t)g.K + 16u * (p & 7);
     }
 #pragma unroll
     for (int i = 0; i < XPT; i++) {
         const int p = tid + i * GT, row = BM * 4 % GT == 0 || p < BM * 4 ? p >> 2 : 0;
         const int m = m0 + row < g.M ? row : g.M - 1 - m0;
-        xoff[i] = (uint32_t)m * (uint32_t)nb + (p & 3);
+        xoff[i] = (uint32_t)arow(m) * (uint32_t)nb + (p & 3);
     }
 #pragma unroll
     for (int i = 0; i < WPT; i++) {
@@ -541,6 +567,8 @@ gemm_i8t(I8tArgs g) {
 
     // While stage s computes from one LDS buffer, stage s + 1 is loaded into
     // registers and then written to the other.
+    // a wave whose token tile is past the group's pairs only stages
+    const bool busy = !MOE || WM == 1 || wm * MT * 32 < g.M;
     // Group kg takes the pairs kg, kg + WK, .. of stages.
     load(2 * kg);
     store(2 * kg, lds);
@@ -548,7 +576,7 @@ gemm_i8t(I8tArgs g) {
     auto stage = [&](auto first, int next) {
         constexpr bool FIRST = decltype(first)::value;
         load(next);
-        compute(first, lds + (FIRST || NBUF == 1 ? 0 : L::bytes));
+        if (busy) compute(first, lds + (FIRST || NBUF == 1 ? 0 : L::bytes));
         if constexpr (NBUF == 1) __builtin_amdgcn_wave_barrier();
         store(next, lds + (FIRST && NBUF == 2 ? L::bytes : 0));
         if constexpr (NBUF == 1) __builtin_amdgcn_wave_barrier();
@@ -560,12 +588,12 @@ gemm_i8t(I8tArgs g) {
         // few stages per group: the last one does not wait for a load nobody needs
         // (the same call 11.6 -> 11.0 us)
         if (WK > 1 && it == iters - 1) {
-            compute(Flag<false>{}, lds + (NBUF == 1 ? 0 : L::bytes));
+            if (busy) compute(Flag<false>{}, lds + (NBUF == 1 ? 0 : L::bytes));
             flush();
             break;
         }
         stage(Flag<false>{}, s + 2 * WK);
-        flush();
+        if (busy) flush();
     }
     if constexpr (WK > 1) {
         __syncthreads();      // every wave is done with its buffer
@@ -588,7 +616,7 @@ gemm_i8t(I8tArgs g) {
             const int i = j & 15, n = n0 + (wn * NT + (j >> 4) % NT) * 32 + col;
             const int m = m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
             if (m < g.M && n < g.N) {
-                g.y[(size_t)m * g.N + n] = (float)u;
+                g.y[yrow(m) + n] = (float)u;
             }
         }
         return;
@@ -601,21 +629,21 @@ gemm_i8t(I8tArgs g) {
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int m = m0 + (wm * MT + t) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (m < g.M && n < g.N) g.y[(size_t)m * g.N + n] = (float)sum[t][r][i];
+                if (m < g.M && n < g.N) g.y[yrow(m) + n] = (float)sum[t][r][i];
             }
     }
 }
 
-template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
+template <uint32_t T, int MT, int NT, int WM, int WN, int WK, bool MOE = false>
 hipError_t launch_cfg(I8tArgs g, hipStream_t st) {
     constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
     constexpr int red = WK > 1 ? WK * WM * WN * MT * NT * 8192 : 0;
     constexpr int bufs = WK * (WM * WN == 1 ? 1 : 2) * Lay<T, BM, BN>::bytes;
     constexpr int lds = bufs > red ? bufs : red;
     static_assert(lds <= 160 * 1024, "LDS");
-    g.ntm = (g.M + BM - 1) / BM;
+    if (!MOE) g.ntm = (g.M + BM - 1) / BM;
     g.ntn = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((gemm_i8t<T, MT, NT, WM, WN, WK>), dim3((unsigned)(g.ntm * g.ntn)), dim3(64 * WM * WN * WK), lds,
+    hipLaunchKernelGGL((gemm_i8t<T, MT, NT, WM, WN, WK, MOE>), dim3((unsigned)(g.ntm * g.ntn)), dim3(64 * WM * WN * WK), lds,
                        st, g);
     return hipGetLastError();
 }
@@ -707,7 +735,7 @@ bool i8t_preferred(uint32_t type, int M, int K, int N) {
 hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
                            hipStream_t st) {
     if (M <= 0 || N <= 0) return hipSuccess;
-    const I8tArgs g{w, A, y, M, N, K, row_bytes(type, K), 0, 0};
+    I8tArgs g{w, A, y, M, N, K, row_bytes(type, K)};
     const Form f = pick_form(type, M, N);
     switch (type) {
         case T_Q8_0: return launch_t<T_Q8_0>(g, f, st);
@@ -715,6 +743,57 @@ hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, fl
         case T_Q5_0: return launch_t<T_Q5_0>(g, f, st);
         case T_Q4_K: return launch_t<T_Q4_K>(g, f, st);
         case T_Q6_K: return launch_t<T_Q6_K>(g, f, st);
+    }
+    return hipErrorInvalidValue;
+}
+
+// Grouped MoE: groups of up to 32 / 64 / 128 pairs, one token tile each, on 32 x 128,
+// 64 x 64 and 128 x 128 tiles. A larger group decodes the expert's weights less often
+// and leaves more of its last tile empty. Measured (us, 128 experts, K 2048, N 1536, by
+// pairs per expert; groups of 32 / 64 / 128): Q4_K 19: 95 / 133 / 195, 25: 113 / 146 /
+// 209, 40: 172 / 155 / 208, 62: 221 / 213 / 235, 94: 306 / 297 / 260, 187: 543 / 496 /
+// 458; Q8_0 10: 122 / 124, 25: 152 / 142, 62: 235 / 202 / 236, 131: 392 / 336 / 378;
+// Q6_K 25: 148 / 201, 40: 223 / 219, 62: 287 / 304 / 331, 94: 390 / 419 / 351.
+// Against the kernels for few pairs per expert (us, quantizer and route included): Q4_K
+// groups of 8 at 6 pairs per expert 75 against 92 here, groups of 16 (replaced) at 10 122
+// against 92, at 62 492 against 217; Q8_0 groups of 4 at 2 108 against 113, at 3 142
+// against 117, at 62 2198 against 207; Q6_K at 3 182 against 111. K 14336, N 4096, 8
+// experts, Q4_K at 10 161 against 131.
+int moe_i8t_group(uint32_t type, int rows, int K, int P, int E) {
+    const bool small = type == T_Q8_0 || type == T_Q4_0;
+    if (!(small || type == T_Q4_K || type == T_Q6_K)) return 0;
+    if (type == T_Q4_K ? P <= 8 * (long)E : P < 3 * (long)E) return 0;
+    if ((long)rows * K > 0xffffffffL) return 0;             // 32-bit activation offsets
+    if (P < (small ? 16 : 32) * (long)E) return 32;
+    return small || P <= 80 * (long)E ? 64 : 128;
+}
+
+namespace {
+template <uint32_t T>
+hipError_t launch_moe_t(const I8tArgs& g, int gsize, hipStream_t st) {
+    switch (gsize) {
+        case 32: return launch_cfg<T, 1, 1, 1, 4, 1, true>(g, st);
+        case 64: return launch_cfg<T, 1, 1, 2, 2, 1, true>(g, st);
+        case 128: return launch_cfg<T, 2, 1, 2, 4, 1, true>(g, st);
+    }
+    return hipErrorInvalidValue;
+}
+}  // namespace
+
+hipError_t launch_moe_i8t(uint32_t type, const uint8_t* w, const ActView& A, const void* route, int max_groups,
+                          int gsize, int P, int E, int multi, int topk, float* y, int K, int N, hipStream_t st) {
+    I8tArgs g{w, A, y, 0, N, K, row_bytes(type, K)};
+    g.ntm = P / gsize + (P < E ? P : E);                    // sum over experts of ceil(c / gsize) at most
+    g.route = static_cast<const uint8_t*>(route);
+    g.mg = max_groups;
+    g.multi = multi;
+    g.topk = topk;
+    g.ebytes = (long)g.rb * N;
+    switch (type) {
+        case T_Q8_0: return launch_moe_t<T_Q8_0>(g, gsize, st);
+        case T_Q4_0: return launch_moe_t<T_Q4_0>(g, gsize, st);
+        case T_Q4_K: return launch_moe_t<T_Q4_K>(g, gsize, st);
+        case T_Q6_K: return launch_moe_t<T_Q6_K>(g, gsize, st);
     }
     return hipErrorInvalidValue;
 }

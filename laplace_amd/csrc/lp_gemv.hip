@@ -1903,7 +1903,7 @@ hipError_t launch_gemv(uint32_t type, const uint8_t* w, const ActView& A, float*
 // writes output row p.
 
 constexpr int kMoeGroup = 4;        // pairs per group (GEMV M)
-constexpr int kMoeGroupMf = 16;     // pairs per group on the small-M MFMA kernel (Q4_K)
+constexpr int kMoeGroupTile = 32;   // and more: on the tiled int8 product
 constexpr int kRouteThreads = 1024;
 
 // Route table in the workspace: [count: 1 int][pad to 16 B][groups:
@@ -2025,10 +2025,8 @@ hipError_t launch_moe_grouped_routed(uint32_t type, const uint8_t* w, const ActV
     if (P <= 0 || N <= 0) return hipSuccess;
     if (gu && !moe_geglu_fusable(type, K, gsize, w)) return hipErrorInvalidValue;
     const int mg = moe_max_groups(P, E);
-    if (gsize == kMoeGroupMf) {
-        if (!moe_mf_supported(type, K)) return hipErrorInvalidValue;
-        return launch_moe_i8mf(w, A, route, mg, multi, topk, y, K, N, st);
-    }
+    if (gsize >= kMoeGroupTile)
+        return launch_moe_i8t(type, w, A, route, mg, gsize, P, E, multi, topk, y, K, N, st);
     if (gsize == kRqMoeGroup) {
         if (!rq_moe_supported(type, K)) return hipErrorInvalidValue;
         return launch_moe_rq(w, A, route, mg, gsize, multi, topk, y, K, N, st, gu);

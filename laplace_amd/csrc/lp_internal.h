@@ -153,16 +153,16 @@ hipError_t launch_gemm_planes(uint32_t type, const uint8_t* w, void* planes, flo
 // planes from quantized activations A, then the product
 hipError_t launch_gemm(uint32_t type, const uint8_t* w, const ActView& A, void* planes, float* y,
                        int M, int K, int N, hipStream_t st);
-// grouped MoE on the int8 small-M MFMA kernel (groups of <= 16 pairs) from
-// the quantized activation rows A; route from launch_moe_route with group
-// size 16.
-bool moe_mf_supported(uint32_t type, int K);
-hipError_t launch_moe_i8mf(const uint8_t* w, const ActView& A, const void* route, int max_groups, int multi,
-                           int topk, float* y, int K, int N, hipStream_t st);
+// grouped MoE on the tiled int8 product (lp_gemm_i8t.hip): the group size (32, 64,
+// 128) where P pairs on E experts run on it, else 0; route from launch_moe_route with
+// that group size.
+int moe_i8t_group(uint32_t type, int rows, int K, int P, int E);
+hipError_t launch_moe_i8t(uint32_t type, const uint8_t* w, const ActView& A, const void* route, int max_groups,
+                          int gsize, int P, int E, int multi, int topk, float* y, int K, int N, hipStream_t st);
 // Grouped MoE dispatch (lp_gemv.hip). P = T * topk pairs, E experts stacked
 // in w (E x N rows). `route` is scratch of moe_route_bytes(P, E) bytes.
 // gsize: pairs per group (the group is the activation-row count of one
-// workgroup): 16 for the 16x16 int8 MFMA kernel (Q4_K), 8 for the row-quad
+// workgroup): 32 and more for the tiled int8 product (moe_i8t_group), 8 for the row-quad
 // kernel (Q4_K, rq_moe_supported), 4 for the GEMV kernels (any type; Q4_K on
 // the row-quad kernel where supported).
 constexpr int kMoeMaxExperts = 8192;
