@@ -71,11 +71,17 @@ struct Q6Tile {
     uint32_t sh;         // byte offset of the block start in dword 0 (0 or 2)
 };
 
-template <int TG, bool COAL>
+// ONE: one token. It alone is staged and stands in all four rows of A, of whose
+// sums only the first is used: a quarter of the staging, LDS and fma work of short-lived
+// workgroups that are otherwise bound by the weight stream (us, N 262144 K 2816 144 ->
+// 136, 151936 x 3584 102 -> 97.5, 14336 x 4096 14.1 -> 13.9, 4096 x 4096 8.8; the
+// same bits). With 5 waves per SIMD instead of 4 (launch bounds) 142, and the weights
+// requested before the staging barrier 150.
+template <int TG, bool COAL, bool ONE = false>
 __global__ void __launch_bounds__(64 * kQ6rqWaves)
 gemv_q6k_rq(Q6rqArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    constexpr int MP = 4 * TG;
+    constexpr int MP = ONE ? 1 : 4 * TG;
     constexpr int SS = 96 * TG + 4;           // dwords per super-block of block scales
     const int K = a.K, N = a.N, M = a.M;
     const int nsb = K >> 8, nb = K >> 5;
@@ -107,8 +113,8 @@ gemv_q6k_rq(Q6rqArgs a) {
     };
 
     // chunk staging: tokens' codes (16-byte pieces) and per block xd, c0, c1
-    constexpr int PPT = MP * 256 / (64 * kQ6rqWaves);      // code pieces per thread
-    constexpr int BPT = MP * 128 / (64 * kQ6rqWaves);      // blocks per thread
+    constexpr int PPT = MP * 256 / (64 * kQ6rqWaves);                             // code pieces per thread
+    constexpr int BPT = (MP * 128 + 64 * kQ6rqWaves - 1) / (64 * kQ6rqWaves);     // blocks per thread
     u32x4 sp[PPT];
     float sxd[BPT];
     int sc0[BPT], sc1[BPT];
@@ -152,6 +158,7 @@ gemv_q6k_rq(Q6rqArgs a) {
         for (int k = 0; k < BPT; k++) {
             const int i = threadIdx.x + 64 * kQ6rqWaves * k;
             const int m = i >> 7, bl = i & 127;
+            if (ONE && m >= MP) break;
             const int o = (bl >> 3) * SS + (bl & 7) * 12 * TG + 12 * (m >> 2) + (m & 3);
             sx[o] = __float_as_int(sxd[k]);
             sx[o + 4] = sc0[k];
@@ -181,7 +188,7 @@ gemv_q6k_rq(Q6rqArgs a) {
         const float d = qv ? fp16_bits_to_f32(dh) : 0.0f;
         const uint8_t* codes = smem + (size_t)buf * a.buf_bytes;
         const int* sx = reinterpret_cast<const int*>(codes + MP * kQ6rqTok) + q * SS;
-        const uint8_t* aq = codes + j * kQ6rqTok + q * 272;
+        const uint8_t* aq = codes + (ONE ? 0 : j * kQ6rqTok) + q * 272;
         f4v acc[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) acc[t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
@@ -207,9 +214,9 @@ gemv_q6k_rq(Q6rqArgs a) {
                         const u32x4 a0 = *reinterpret_cast<const u32x4*>(at);
                         const u32x4 a1 = *reinterpret_cast<const u32x4*>(at + 16);
                         const int* bs = sx + g * 12 * TG + 12 * t;
-                        const f4v xd = *reinterpret_cast<const f4v*>(bs);
-                        i4v p0 = *reinterpret_cast<const i4v*>(bs + 4);
-                        i4v p1 = *reinterpret_cast<const i4v*>(bs + 8);
+                        const f4v xd = ONE ? f4v{*reinterpret_cast<const float*>(bs), 0, 0, 0} : *reinterpret_cast<const f4v*>(bs);
+                        i4v p0 = ONE ? i4v{bs[4], 0, 0, 0} : *reinterpret_cast<const i4v*>(bs + 4);
+                        i4v p1 = ONE ? i4v{bs[8], 0, 0, 0} : *reinterpret_cast<const i4v*>(bs + 8);
                         p0 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a0.x, (int)v[0], p0, 0, 0, 0);
                         p0 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a0.y, (int)v[1], p0, 0, 0, 0);
                         p0 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a0.z, (int)v[2], p0, 0, 0, 0);
@@ -219,7 +226,7 @@ gemv_q6k_rq(Q6rqArgs a) {
                         p1 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a1.z, (int)v[6], p1, 0, 0, 0);
                         p1 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a1.w, (int)v[7], p1, 0, 0, 0);
 #pragma unroll
-                        for (int r = 0; r < 4; r++) {
+                        for (int r = 0; r < (ONE ? 1 : 4); r++) {
                             const int I = __mul24(s0, p0[r]) + __mul24(s1, p1[r]);
                             acc[t][r] = fmaf((float)I, xd[r], acc[t][r]);
                         }
@@ -231,7 +238,7 @@ gemv_q6k_rq(Q6rqArgs a) {
 #pragma unroll
         for (int t = 0; t < TG; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) tot[t][r] = fmaf(d, acc[t][r], tot[t][r]);
+            for (int r = 0; r < (ONE ? 1 : 4); r++) tot[t][r] = fmaf(d, acc[t][r], tot[t][r]);
     };
 
     const int nc = a.nchunk;
@@ -378,7 +385,9 @@ q6rq_reduce(const float* __restrict__ part, int nsplit, long mn, float* __restri
 
 static int q6rq_tg(int M) { return M <= 4 ? 1 : 2; }
 
-static size_t q6rq_buf(int TG) { return (size_t)4 * TG * kQ6rqTok + (size_t)16 * (96 * TG + 4) * 4; }
+static size_t q6rq_buf(int TG, bool one = false) {
+    return (size_t)(one ? 1 : 4 * TG) * kQ6rqTok + (size_t)16 * (96 * TG + 4) * 4;
+}
 
 bool q6rq_supported(uint32_t type, int M, int K, int N, const uint8_t* w) {
     // w 4-byte aligned: a block at byte 2 of a dword is read from the dword below it
@@ -421,7 +430,9 @@ hipError_t launch_gemv_q6rq(const uint8_t* w, const ActView& A, float* y, int M,
     const dim3 grid((unsigned)gx, split ? (unsigned)a.nchunk : 1u);
     const size_t shm = coal ? 2 * q6rq_buf(TG) + (size_t)kQ6rqWaves * 4 * kQ6rqRowStride : q6rq_buf(TG);
 #define LP_Q6RQ_LAUNCH(TGV, CV) hipLaunchKernelGGL((gemv_q6k_rq<TGV, CV>), grid, dim3(64 * kQ6rqWaves), shm, st, a)
-    if (TG == 1) {
+    if (M == 1 && !coal) {
+        hipLaunchKernelGGL((gemv_q6k_rq<1, false, true>), grid, dim3(64 * kQ6rqWaves), q6rq_buf(1, true), st, a);
+    } else if (TG == 1) {
         if (coal) LP_Q6RQ_LAUNCH(1, true);
         else LP_Q6RQ_LAUNCH(1, false);
     } else {
