@@ -696,7 +696,7 @@ int lp_gemm_dev(const float* x, const uint8_t* w, uint32_t type, float* y, int M
     int rc = check_shape(type, w, M, K, N);
     if (rc != LP_OK) return rc;
     if (fact_type(type)) {
-        // fp32 activations straight into the GEMV (no workspace)
+        // fp32 activations straight into the kernels (no workspace)
         if (M > 0 && N > 0 && (!x || !y)) {
             set_err("null pointer");
             return LP_EINVAL;

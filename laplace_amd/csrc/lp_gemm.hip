@@ -986,28 +986,22 @@ __device__ __forceinline__ uint2 ld8_a2(const uint8_t* p) {
     return make_uint2((d0 >> 16) | (d1 << 16), (d1 >> 16) | (t << 16));
 }
 
-template <int TL, int NWV, int TT = 1>
+template <int TL, int NWV>
 __global__ void __launch_bounds__(64 * NWV)
 gemv_q6k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restrict__ y, int M, int K, int N) {
-    static_assert(TL * TT <= NWV, "one wave per output tile in the final sum");
-    constexpr int TK = 16 * TT;                  // tokens per workgroup (TT 16-token tiles)
-    __shared__ f4v red[NWV][TL * TT][64];
-    extern __shared__ __attribute__((aligned(16))) float sdx[];   // [nb][TK] xd
+    static_assert(TL <= NWV, "one wave per output tile in the final sum");
+    __shared__ f4v red[NWV][TL][64];
+    extern __shared__ __attribute__((aligned(16))) float sdx[];   // [nb][16] xd
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int tok = lane & 15, g = lane >> 4;
     const int nsb = K >> 8, nb = K >> 5;
-    for (int i = threadIdx.x; i < nb * TK; i += blockDim.x) {
-        const int b = i / TK, t = i % TK;
+    for (int i = threadIdx.x; i < nb * 16; i += blockDim.x) {
+        const int b = i >> 4, t = i & 15;
         sdx[i] = t < M ? A.d[(size_t)t * nb + b] : 0.0f;
     }
     __syncthreads();
-    bool tv[TT];
-    const int8_t* aq[TT];
-#pragma unroll
-    for (int u = 0; u < TT; u++) {
-        tv[u] = tok + 16 * u < M;
-        aq[u] = A.qs + (size_t)(tv[u] ? tok + 16 * u : 0) * K + 8 * g;
-    }
+    const bool tv = tok < M;
+    const int8_t* aq = A.qs + (size_t)(tv ? tok : 0) * K + 8 * g;
     const int row0 = blockIdx.x * (16 * TL) + (lane & 15);
     const int sb0 = wv * nsb / NWV, sb1 = (wv + 1) * nsb / NWV;
     const uint8_t* wr[TL];
@@ -1020,11 +1014,9 @@ gemv_q6k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restri
     const bool first_half = g < 2;                 // k 0..15 of the block
     const i4v zi = {0, 0, 0, 0};
     const f4v z4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    f4v acc[TL][TT];
+    f4v acc[TL];
 #pragma unroll
-    for (int t = 0; t < TL; t++)
-#pragma unroll
-        for (int u = 0; u < TT; u++) acc[t][u] = z4;
+    for (int t = 0; t < TL; t++) acc[t] = z4;
     for (int s = sb0; s < sb1; s++) {
         uint2 ql[TL][4], qh[TL][2];
         uint32_t scw[TL][4];
@@ -1040,12 +1032,9 @@ gemv_q6k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restri
             scw[t][0] = s0.x; scw[t][1] = s0.y; scw[t][2] = s1.x; scw[t][3] = s1.y;
             d[t] = fp16_bits_to_f32(*reinterpret_cast<const uint16_t*>(blk + 208));
         }
-        long av[TT][8];
+        long av[8];
 #pragma unroll
-        for (int u = 0; u < TT; u++)
-#pragma unroll
-            for (int b = 0; b < 8; b++)
-                av[u][b] = tv[u] ? *reinterpret_cast<const long*>(aq[u] + 32 * (8 * s + b)) : 0L;
+        for (int b = 0; b < 8; b++) av[b] = tv ? *reinterpret_cast<const long*>(aq + 32 * (8 * s + b)) : 0L;
 #pragma unroll
         for (int b = 0; b < 8; b++) {
             const int h = b >> 2, g6 = b & 3;
@@ -1063,37 +1052,31 @@ gemv_q6k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restri
                 const int si = 8 * h + 2 * g6;          // scales of the block's two halves
                 const float sc0 = (float)(int8_t)(scw[t][si >> 2] >> (8 * (si & 3)));
                 const float sc1 = (float)(int8_t)(scw[t][(si + 1) >> 2] >> (8 * ((si + 1) & 3)));
+                const f4v xd = *reinterpret_cast<const f4v*>(sdx + (size_t)(8 * s + b) * 16 + 4 * g);
+                const i4v S0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[b], b0, zi, 0, 0, 0);
+                const i4v S1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[b], b1, zi, 0, 0, 0);
 #pragma unroll
-                for (int u = 0; u < TT; u++) {
-                    const f4v xd = *reinterpret_cast<const f4v*>(sdx + (size_t)(8 * s + b) * TK + 16 * u + 4 * g);
-                    const i4v S0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[u][b], b0, zi, 0, 0, 0);
-                    const i4v S1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[u][b], b1, zi, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float dx = d[t] * xd[r];
-                        acc[t][u][r] = fmaf(dx * sc0, (float)S0[r], acc[t][u][r]);
-                        acc[t][u][r] = fmaf(dx * sc1, (float)S1[r], acc[t][u][r]);
-                    }
+                for (int r = 0; r < 4; r++) {
+                    const float dx = d[t] * xd[r];
+                    acc[t][r] = fmaf(dx * sc0, (float)S0[r], acc[t][r]);
+                    acc[t][r] = fmaf(dx * sc1, (float)S1[r], acc[t][r]);
                 }
             }
         }
     }
 #pragma unroll
-    for (int t = 0; t < TL; t++)
-#pragma unroll
-        for (int u = 0; u < TT; u++) red[wv][t * TT + u][lane] = acc[t][u];
+    for (int t = 0; t < TL; t++) red[wv][t][lane] = acc[t];
     __syncthreads();
-    // wave i sums output tile i (row tile i / TT, token tile i % TT)
-    if (wv < TL * TT) {
-        const int t = wv / TT, u = wv % TT;
+    // wave i sums output tile i
+    if (wv < TL) {
         f4v sum = red[0][wv][lane];
 #pragma unroll
         for (int i = 1; i < NWV; i++) sum += red[i][wv][lane];
-        const int row = row0 + 16 * t;
+        const int row = row0 + 16 * wv;
         if (row < N) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int tt = 16 * u + 4 * g + r;
+                const int tt = 4 * g + r;
                 if (tt < M) y[(size_t)tt * N + row] = sum[r];
             }
         }
