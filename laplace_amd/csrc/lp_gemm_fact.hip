@@ -553,10 +553,6 @@ hipError_t launch_cfg(FactArgs g, hipStream_t st) {
 
 }  // namespace
 
-#ifdef LP_DEV
-int g_fact_cfg = -1;
-#endif
-
 namespace {
 // The tile forms (as the int8 product's; 64 x 128 where the planes of the weights
 // leave no LDS for 128 x 128). Measured, us, N 4096 K 4096:
@@ -571,9 +567,6 @@ enum Form { F32X32X8, F32X32X4, F64X64X2, F64X64, F64X128, F128X128 };
 
 template <uint32_t T>
 Form pick_form(int M, int N) {
-#ifdef LP_DEV
-    if (g_fact_cfg >= 0) return (Form)g_fact_cfg;
-#endif
     const long cus = device_cu_count();
     auto tiles = [&](int b) { return (long)((M + b - 1) / b) * ((N + b - 1) / b); };
     constexpr bool one = Traits<T>::kPlanes == 1;
@@ -633,11 +626,3 @@ hipError_t launch_gemm_fact(uint32_t type, const uint8_t* w, const float* x, flo
 }
 
 }  // namespace lp
-
-#ifdef LP_DEV
-extern "C" int lp_dev_fact(int cfg, const float* x, const uint8_t* w, uint32_t type, float* y, int M, int K, int N,
-                           unsigned long rb, void* stream) {
-    lp::g_fact_cfg = cfg;
-    return (int)lp::launch_gemm_fact(type, w, x, y, M, K, N, (hipStream_t)stream);
-}
-#endif

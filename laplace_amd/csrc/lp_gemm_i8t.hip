@@ -650,10 +650,6 @@ hipError_t launch_cfg(I8tArgs g, hipStream_t st) {
 
 }  // namespace
 
-#ifdef LP_DEV
-int g_i8t_cfg = -1;
-#endif
-
 namespace {
 // The tile forms, most parallel first. Measured (us per product, CUs 256, K 4096
 // unless said; t32 / t64 / t128 are the tile counts):
@@ -666,9 +662,6 @@ namespace {
 enum Form { F32X32X8, F32X32X4, F64X64X2, F64X64, F128X128 };
 
 Form pick_form(uint32_t type, int M, int N) {
-#ifdef LP_DEV
-    if (g_i8t_cfg >= 0) return (Form)g_i8t_cfg;
-#endif
     const long cus = device_cu_count();
     auto tiles = [&](int b) { return (long)((M + b - 1) / b) * ((N + b - 1) / b); };
     // one 32 x 32 tile per CU: eight waves share its K; two per CU (or at most
@@ -799,13 +792,3 @@ hipError_t launch_moe_i8t(uint32_t type, const uint8_t* w, const ActView& A, con
 }
 
 }  // namespace lp
-
-#ifdef LP_DEV
-extern "C" int lp_dev_i8t(int cfg, const int8_t* qs, const float* d, const float* sum, const uint8_t* w, uint32_t type,
-                          float* y, int M, int K, int N, void* stream) {
-    lp::ActView A;
-    A.qs = const_cast<int8_t*>(qs); A.d = const_cast<float*>(d); A.sum = const_cast<float*>(sum); A.s16 = nullptr;
-    lp::g_i8t_cfg = cfg;
-    return (int)lp::launch_gemm_i8t(type, w, A, y, M, K, N, (hipStream_t)stream);
-}
-#endif
