@@ -160,19 +160,33 @@ __device__ __forceinline__ float hi16(float v) { return __uint_as_float(__float_
 // The operands of a scale product x (x) w on v_mfma_f32_32x32x8_bf16 (4 K slots
 // for lanes < 32, 4 for the others), from the exact bf16 pieces x = x1 + x2 + x3
 // and w = w1 + w2 (an fp16 value) or w1 + w2 + w3 (an fp16 value times a 6-bit
-// one). Two pieces:   x1 x1 x2 x2 . w1 w2 w1 w2 | x3 x3 0 0 . w1 w2 w1 w2
-//          three:     x1 x1 x1 x2 . w1 w2 w3 w1 | x2 x2 x3 x3 . w2 w3 w1 w2
+// one). bf16 ends at 2^-133, fp32 at 2^-149: x2 and x3 are held times 2^13 (x is at
+// most 2^121.01, a 127th of an fp32 value) beside w times 2^-13, w', so that every x
+// from 2^-123 up has its 24 bits (unscaled pieces of x 2^-126 kept 8) and a subnormal
+// one those from 2^-146 up. Two pieces:
+//                      x1 x1 x2 x2 . w1 w2 w1' w2' | 0 0 x3 x3 . w1 w2 w1' w2'
+//          three:     x1 x1 x1 x2 . w1 w2 w3 w1' | x2 x2 x3 x3 . w2' w3' w1' w2'
 // (all products but x3 w3, below 2^-32 of the whole). LDS holds them ready made,
 // 8 bytes per lane.
+constexpr float kUp = 0x1p13f;
+constexpr uint32_t kDown = (13u << 7) * 0x00010001u;
+constexpr float kMinUp = 0x1p6f;                          // of the Q4_K mins' product, its
+constexpr uint32_t kMinDown = 6u << 23;                   // upper halves only
+// Two bf16 divided by powers of two: their exponents less than they are by the halves
+// of k, zeros left (the saturated difference; no piece here is below 2^-64).
+__device__ __forceinline__ uint32_t down(uint32_t v, uint32_t k) {
+    typedef unsigned short h2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(h2, v), __builtin_bit_cast(h2, k)));
+}
 template <int PIECES>
 __device__ __forceinline__ void put_x(u32x2* lo, u32x2* hi, float x) {
-    const float x1 = hi16(x), r = x - x1, x2 = hi16(r), x3 = r - x2;
+    const float x1 = hi16(x), r = (x - x1) * kUp, x2 = hi16(r), x3 = r - x2;
     if constexpr (PIECES == 3) {
         *lo = u32x2{pk_hi(x1, x1), pk_hi(x1, x2)};
         *hi = u32x2{pk_hi(x2, x2), pk_hi(x3, x3)};
     } else {
         *lo = u32x2{pk_hi(x1, x1), pk_hi(x2, x2)};
-        *hi = u32x2{pk_hi(x3, x3), 0u};
+        *hi = u32x2{0u, pk_hi(x3, x3)};
     }
 }
 template <int PIECES>
@@ -180,11 +194,12 @@ __device__ __forceinline__ void put_w(u32x2* lo, u32x2* hi, float w) {
     const float w1 = hi16(w), r = w - w1;
     if constexpr (PIECES == 3) {
         const float w2 = hi16(r), w3 = r - w2;
-        *lo = u32x2{pk_hi(w1, w2), pk_hi(w3, w1)};
-        *hi = u32x2{pk_hi(w2, w3), pk_hi(w1, w2)};
+        const uint32_t p = pk_hi(w1, w2), q = down(p, kDown);
+        *lo = u32x2{p, __builtin_amdgcn_perm(q, __float_as_uint(w3), 0x05040302u)};
+        *hi = u32x2{down(pk_hi(w2, w3), kDown), q};
     } else {
-        const uint32_t v = pk_hi(w1, r);
-        *lo = u32x2{v, v};
+        const uint32_t p = pk_hi(w1, r);
+        *lo = u32x2{p, down(p, kDown)};
     }
 }
 
@@ -527,7 +542,8 @@ gemm_i8t(I8tArgs g) {
         }
         if constexpr (R::kMin) {
             // sum over the stage's four blocks of m * xs: K slots of lane half h
-            // are blocks 2h, 2h + 1, three pieces of xs each
+            // are blocks 2h, 2h + 1, three pieces of xs each, the second and third
+            // times 2^6 beside m' = m times 2^-6 (as x2 and x3 of put_x; xs goes up to 2^128)
             const float* xs = reinterpret_cast<const float*>(st + L::xs) + wm * MT * 32 + col;
             const float* mn = reinterpret_cast<const float*>(st + L::ex) + wn * NT * 32 + col;
             const float* dm = reinterpret_cast<const float*>(st + L::dm) + wn * NT * 32 + col;
@@ -538,7 +554,7 @@ gemm_i8t(I8tArgs g) {
 #pragma unroll
                 for (int u = 0; u < 2; u++) {
                     const float x = xs[(2 * half + u) * BM + 32 * t];
-                    const float x1 = hi16(x), q = x - x1, x2 = hi16(q);
+                    const float x1 = hi16(x), q = (x - x1) * kMinUp, x2 = hi16(q);
                     o[2 * u] = pk_hi(x1, x2);
                     o[2 * u + 1] = pk_hi(q - x2, 0.0f);
                 }
@@ -550,8 +566,8 @@ gemm_i8t(I8tArgs g) {
 #pragma unroll
                 for (int u = 0; u < 2; u++) {
                     const float m = mn[(2 * half + u) * BN + 32 * r];
-                    o[2 * u] = pk_hi(m, m);
-                    o[2 * u + 1] = pk_hi(m, 0.0f);
+                    o[2 * u] = down(pk_hi(m, m), kMinDown);
+                    o[2 * u + 1] = o[2 * u] >> 16;
                 }
                 const b8v mb = __builtin_bit_cast(b8v, o);
                 const float nd = -dm[32 * r];

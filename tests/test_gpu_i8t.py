@@ -3,7 +3,7 @@ small-M kernels) at the edges of its tiles and forms, against the oracle."""
 import numpy as np
 import pytest
 
-from hip_util import L, gemm_dev, normwise, synth_weights, synth_x, to_dev
+from hip_util import L, gemm_dev, normwise, quantize_dev, synth_weights, synth_x, to_dev
 from oracle.oracle import Q4_0, Q4_K, Q5_0, Q6_K, Q8_0
 
 pytestmark = pytest.mark.gpu
@@ -77,3 +77,49 @@ def test_i8t_non_finite_rows(orc, t):
     assert np.array_equal(np.isnan(y), np.isnan(ref))
     good = [m for m in range(M) if m not in (3, 68, 69)]
     assert normwise(y[good], ref[good]) <= TOL
+
+
+# each form, K ending inside a stage where the type allows it
+EDGE_SHAPES = [(9, 600, 192), (40, 8200, 192), (96, 4300, 320), (70, 14400, 192), (257, 16390, 192)]
+
+
+@pytest.mark.parametrize("wscale", [None, 2.0 ** -24, 6e4])
+@pytest.mark.parametrize("M,N,K", EDGE_SHAPES)
+@pytest.mark.parametrize("t", list(NAMES), ids=list(NAMES.values()))
+def test_i8t_tiny_rows(orc, t, M, N, K, wscale):
+    """Rows down to the smallest fp32 values keep their products' 24 bits, whatever the
+    block scales of the weights; the rows beside them keep their bits."""
+    print(f"i8t tiny rows {NAMES[t]} M={M} N={N} K={K}", flush=True)
+    if t in (Q4_K, Q6_K):
+        K, M = 512, max(M, 17 if t == Q6_K else 70)
+    if t == Q4_K and M > 200:                              # one round of 128 x 128 tiles
+        M, N = 130, 16300
+    w = weights(t, K, N, seed=t).reshape(-1, {Q8_0: 34, Q4_0: 18, Q5_0: 22, Q4_K: 144, Q6_K: 210}[t])
+    for at in {Q4_K: [0, 2], Q6_K: [208]}.get(t, [0]):
+        if wscale:
+            w[:, at:at + 2] = np.array([wscale], np.float16).view(np.uint8)
+    w = w.reshape(-1)
+    x = synth_x(M, K, seed=32)
+    plain = gemm_dev(t, x, w, N)
+    scale = {0: 1e-20, 1: 1e-26, 3: 1e-30, 4: 1e-33, 6: 1e-36, 7: 0.0, M - 1: 1e-31}
+    for m, s in scale.items():
+        x[m] *= np.float32(s)
+    y = gemm_dev(t, x, w, N)
+    d, _, _, qs = quantize_dev(x)
+    X = np.repeat(d.astype(np.float64), 32, axis=1) * qs
+    rows = np.unique(np.linspace(0, N - 1, 64).astype(int))
+    rb = len(w) // N
+    sub = np.concatenate([w[r * rb:(r + 1) * rb] for r in rows])
+    W = orc.dequantize(t, sub, len(rows) * K)
+    ref = X @ W.astype(np.float64).reshape(len(rows), K).T
+    few = list(scale)
+    P = np.abs(orc.block_sums(t, sub, qs[few], K, len(rows))).sum(-1).max(-1)
+    for i, m in enumerate(few):
+        # products of scales below 2^-126 are rounded at 2^-149 (as in fp32), then
+        # multiplied with a block sum (of Q6_K times its int8 scale; of Q4_K the 6-bit
+        # mins' product too, by a factor up to 2^11 of fp16 dmin)
+        quantum = 2.0 ** -149 * (P[i] * (128 if t == Q6_K else 1) + (2048 * K if t == Q4_K else K))
+        err = np.abs(y[m, rows] - ref[m]).max()
+        assert err <= TOL * np.abs(ref[m]).max() + quantum, (m, scale[m], err, np.abs(ref[m]).max())
+    rest = [m for m in range(M) if m not in scale]
+    assert np.array_equal(y[rest].view(np.uint32), plain[rest].view(np.uint32))
