@@ -36,6 +36,7 @@
 // (7.5e-8 normwise against 0.96e-7 at K 4096, 1.8e-7 at K 18944).
 #include <hip/hip_runtime.h>
 
+#include "lp_chunks.h"
 #include "lp_internal.h"
 
 namespace lp {
@@ -311,6 +312,40 @@ __device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, in
         if (c == 0) put_w<2>(wd + n, nullptr, fp16_bits_to_f32(r.d));
     }
 }
+
+// One output by the whole wave in fp32, as the few-row kernels form it. An infinite
+// block scale has no pieces (inf - inf), so its product above is NaN where the plain
+// one is an infinity: non-finite outputs are made again here, except in rows whose
+// own scales are not finite (a NaN or infinite activation), which are NaN either way.
+template <uint32_t T>
+__device__ __forceinline__ float wave_dot(const ActView& A, int arow, const uint8_t* wrow, int K, int lane) {
+    float s = 0.0f;
+    if constexpr (T == T_Q5_0) {
+        const int8_t* q = A.qs + (size_t)arow * K;
+        for (int b = lane; b < K >> 5; b += 64) {
+            const uint8_t* blk = wrow + b * 22;
+            const uint32_t qh = load_u16(blk + 2) | load_u16(blk + 4) << 16;
+            int P = 0;
+            for (int e = 0; e < 32; e++) {
+                const int nib = e < 16 ? blk[6 + e] & 15 : blk[6 + e - 16] >> 4;
+                P += ((nib | (int)((qh >> e) & 1u) << 4) - 16) * q[32 * b + e];
+            }
+            s = fmaf(fp16_bits_to_f32(load_u16(blk)) * A.d[(size_t)arow * (K >> 5) + b], (float)P, s);
+        }
+    } else {
+        for (int c = lane; c < K >> 6; c += 64) {
+            typename Chunk<T>::Act a;
+            typename Chunk<T>::Wt w;
+            int is[Chunk<T>::NSUB];
+            load_act<T>(A, K, arow, c, a);
+            Chunk<T>::load_w(wrow, c, w);
+            Chunk<T>::isums(w, a, is);
+            s += Chunk<T>::partial(w, a, is, c);
+        }
+    }
+    return wave_sum(s);
+}
+__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
 
 // MT x NT tiles of 32 x 32 per wave. MOE: a token tile is a routed group (expert,
 // first pair, n <= BM pairs); its rows are gathered and scattered by pair.
@@ -611,12 +646,23 @@ gemm_i8t(I8tArgs g) {
         stage(Flag<false>{}, s + 2 * WK);
         if (busy) flush();
     }
+    bool bad = false;
+    // register j = (t * NT + r) * 16 + i of a lane: its token and weight row (the lane's
+    // number is read again, so that the part below keeps no register through the loop:
+    // two more than 168 cost a wave per SIMD)
+    const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    auto mrow = [&](int j) { return m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * ((j & 15) >> 2) + 4 * (ln >> 5) + (j & 3); };
+    auto nrow = [&](int j) { return n0 + (wn * NT + (j >> 4) % NT) * 32 + (ln & 31); };
+    auto put = [&](int j, float v) {
+        const int m = mrow(j), n = nrow(j);
+        if (m < g.M && n < g.N) g.y[yrow(m) + n] = v;
+    };
     if constexpr (WK > 1) {
         __syncthreads();      // every wave is done with its buffer
         // All groups leave their sums in LDS; group kg adds those of registers kg,
         // kg + WK, .. in the groups' order (against one group adding the others' one
         // after the other: Q8_0 N 4096 K 4096 M 16 13.1 -> 11.6 us with the quantizer).
-        double* red = reinterpret_cast<double*>(smem) + wave * MT * NT * 16 * 64 + lane;
+        double* red = reinterpret_cast<double*>(smem) + wave * MT * NT * 16 * 64 + ln;
         constexpr int kGrp = WM * WN * MT * NT * 16 * 64;
 #pragma unroll
         for (int t = 0; t < MT; t++)
@@ -629,24 +675,41 @@ gemm_i8t(I8tArgs g) {
             double u = red[j * 64];
 #pragma unroll
             for (int q = 1; q < WK; q++) u += red[q * kGrp + j * 64];
-            const int i = j & 15, n = n0 + (wn * NT + (j >> 4) % NT) * 32 + col;
-            const int m = m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-            if (m < g.M && n < g.N) {
-                g.y[yrow(m) + n] = (float)u;
-            }
+            bad |= !finite((float)u);
+            put(j, (float)u);
         }
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < NT; r++) {
-        const int n = n0 + (wn * NT + r) * 32 + col;
+    } else {
 #pragma unroll
         for (int t = 0; t < MT; t++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int m = m0 + (wm * MT + t) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (m < g.M && n < g.N) g.y[yrow(m) + n] = (float)sum[t][r][i];
-            }
+            for (int r = 0; r < NT; r++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    bad |= !finite((float)sum[t][r][i]);
+                    put((t * NT + r) * 16 + i, (float)sum[t][r][i]);
+                }
+    }
+    // (without the hint the MoE prompt's kernel is laid out worse: 424 -> 459 us a layer)
+    if (__builtin_expect(!__any(bad), 1)) return;
+    for (int j = kg; j < MT * NT * 16; j += WK) {
+        const int m = mrow(j), n = nrow(j);
+        const bool in = m < g.M && n < g.N;
+        float* const y = g.y + (in ? yrow(m) + n : 0);
+        uint64_t left = __ballot(in && !finite(*y));
+        if (!left) continue;
+        // each half's 32 lanes look through the scales of its row
+        bool nan = false;
+        if (m < g.M)
+            for (int b = ln & 31; b < nb; b += 32) nan |= !finite(g.A.d[(size_t)arow(m) * nb + b]);
+        const uint64_t nans = __ballot(nan);
+        if ((uint32_t)nans) left &= ~0xffffffffull;
+        if (nans >> 32) left &= 0xffffffffull;
+        for (; left; left &= left - 1) {
+            const int l = __ffsll((unsigned long long)left) - 1;
+            const int row = __builtin_amdgcn_readlane(n, l);
+            const float v = wave_dot<T>(g.A, arow(__builtin_amdgcn_readlane(m, l)), g.w + (size_t)row * g.rb, g.K, ln);
+            if (ln == l) *y = v;
+        }
     }
 }
 

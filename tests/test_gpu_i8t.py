@@ -123,3 +123,60 @@ def test_i8t_tiny_rows(orc, t, M, N, K, wscale):
         assert err <= TOL * np.abs(ref[m]).max() + quantum, (m, scale[m], err, np.abs(ref[m]).max())
     rest = [m for m in range(M) if m not in scale]
     assert np.array_equal(y[rest].view(np.uint32), plain[rest].view(np.uint32))
+
+
+def positive_weights(t, K, N, seed):
+    """Blocks whose codes and sub-scales are all above zero (every block sum with positive
+    activations is too), mins of the type zero; returns them with a view of the rows'
+    block scales [N, blocks] as fp16 bits."""
+    rng = np.random.default_rng(seed)
+    size, elems, at = {Q8_0: (34, 32, 0), Q4_0: (18, 32, 0), Q5_0: (22, 32, 0), Q4_K: (144, 256, 0), Q6_K: (210, 256, 208)}[t]
+    b = rng.integers(0, 256, (N * (K // elems), size), dtype=np.uint8)
+    n = len(b)
+    nib = lambda lo, hi, w: (rng.integers(lo, hi, (n, w)) | rng.integers(lo, hi, (n, w)) << 4).astype(np.uint8)
+    if t == Q8_0:
+        b[:, 2:] = rng.integers(1, 128, (n, 32))
+    elif t == Q4_0:
+        b[:, 2:] = nib(9, 16, 16)
+    elif t == Q5_0:
+        b[:, 2:6], b[:, 6:] = 255, nib(1, 16, 16)
+    elif t == Q4_K:
+        b[:, 2:4], b[:, 16:] = 0, nib(1, 16, 128)
+        b[:, 4:8], b[:, 8:12], b[:, 12:16] = 0x41, 0, 0x0f      # scales 1 and 31, mins 0
+    else:
+        b[:, :128], b[:, 128:192], b[:, 192:208] = nib(1, 16, 128), 0xaa, rng.integers(1, 32, (n, 16))
+    d = (0.01 * (0.5 + rng.random(n))).astype(np.float16)
+    b[:, at:at + 2] = d.view(np.uint8).reshape(-1, 2)
+    return b, b.reshape(N, -1, size)[:, :, at:at + 2].view(np.uint16)[:, :, 0]
+
+
+@pytest.mark.parametrize("M,N,K", EDGE_SHAPES)
+@pytest.mark.parametrize("t", list(NAMES), ids=list(NAMES.values()))
+def test_i8t_infinite_block_scales(t, M, N, K):
+    """An infinite block scale gives the signed infinity of its product (NaN with a block
+    of zeros, or beside an infinity of the other sign), a NaN scale NaN, as at few rows
+    (whose kernels multiply a row's last block with zeros once more past its end, which is
+    left out here); the other weight rows keep their bits."""
+    print(f"i8t infinite scales {NAMES[t]} M={M} N={N} K={K}", flush=True)
+    if t in (Q4_K, Q6_K):
+        K, M = 512, max(M, 17 if t == Q6_K else 70)
+    if t == Q4_K and M > 200:
+        M, N = 130, 16300
+    x = np.abs(synth_x(M, K, seed=31)) + 0.1
+    x[2] = 0.0
+    w, d = positive_weights(t, K, N, seed=t)
+    clean = gemm_dev(t, x, w.reshape(-1), N)
+    inf, ninf, nan = 0x7c00, 0xfc00, 0x7e00
+    d[4, 0], d[N - 1, -1], d[7, 0], d[7, -1], d[9, 0], d[65, 1] = inf, ninf, inf, ninf, nan, inf
+    want = clean.copy()
+    want[:, [4, 65]], want[:, N - 1], want[:, [7, 9]] = np.inf, -np.inf, np.nan
+    want[2, [4, 65, N - 1]] = np.nan
+    if t == Q4_0:                                          # the reference subtracts 8 d sum(x): inf - inf
+        want[:, [4, 65, N - 1]] = np.nan
+    y = gemm_dev(t, x, w.reshape(-1), N)
+    few = gemm_dev(t, x[:3], w.reshape(-1), N)
+    special = [4, 7, 9, 65, N - 1]
+    assert np.array_equal(few[:, special[:4]], want[:3, special[:4]], equal_nan=True)
+    assert np.array_equal(y[:, special], want[:, special], equal_nan=True)
+    rest = np.setdiff1d(np.arange(N), special)
+    assert np.array_equal(y[:, rest].view(np.uint32), clean[:, rest].view(np.uint32))

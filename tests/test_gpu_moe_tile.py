@@ -5,6 +5,7 @@ import pytest
 
 from hip_util import L, normwise, stream, synth_weights, synth_x, to_dev
 from oracle.oracle import Q4_0, Q4_K, Q6_K, Q8_0
+from test_gpu_i8t import positive_weights
 
 pytestmark = pytest.mark.gpu
 NAMES = {Q8_0: "Q8_0", Q4_0: "Q4_0", Q6_K: "Q6_K", Q4_K: "Q4_K"}
@@ -77,3 +78,27 @@ def test_moe_tile_drops_pairs_without_an_expert(t):
     drop = (bad != idx).reshape(-1)
     assert np.all(y[drop] == 7.0)
     assert np.array_equal(y[~drop].view(np.uint32), want[~drop].view(np.uint32))
+
+
+@pytest.mark.parametrize("multi", [0, 1])
+@pytest.mark.parametrize("gs", list(COUNTS))
+@pytest.mark.parametrize("t", list(NAMES), ids=list(NAMES.values()))
+def test_moe_tile_infinite_block_scales(t, gs, multi):
+    """An infinite block scale of an expert's row gives that expert's pairs the signed
+    infinity (Q4_0, whose offset is subtracted apart, NaN) and no other output another value;
+    a NaN activation row is NaN."""
+    rng = np.random.default_rng(gs)
+    E, K, N, topk = 8, 512, 70, 2
+    idx = pairs_of(COUNTS[gs], topk, rng)
+    P = idx.size
+    x = np.abs(synth_x(P if multi else len(idx), K, seed=6)) + 0.1
+    w, d = positive_weights(t, K, E * N, seed=gs)
+    clean = grouped(t, x, multi, idx, w.reshape(-1), E, K, N)
+    d[2 * N + 3, 0], d[4 * N + N - 1, -1] = 0x7c00, 0xfc00
+    x[1, 7] = np.nan
+    y = grouped(t, x, multi, idx, w.reshape(-1), E, K, N)
+    e = idx.reshape(-1)
+    want = clean.copy()
+    want[e == 2, 3], want[e == 4, N - 1] = (np.nan, np.nan) if t == Q4_0 else (np.inf, -np.inf)
+    want[1 if multi else [topk, topk + 1]] = np.nan
+    assert np.array_equal(y, want, equal_nan=True)
