@@ -235,37 +235,105 @@ __device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, in
     }
 }
 
-// One output in fp32. The pieces of an infinity are (inf, 0, 0) and its product
+// Outputs made again in fp32. The pieces of an infinity are (inf, 0, 0) and its product
 // with a zero piece of a finite value is NaN, so are partial sums past the fp32
 // range with opposite signs, and the matrix unit takes pieces below 2^-126 as zero
 // (third pieces of values below 2^-108). Outputs that come out infinite, NaN or
 // nonzero and below 2^-80 (there by such values, not by cancellation: the 64-bit
-// sums of larger ones end in a whole zero or far above) are computed again so. A
-// NaN sum stays one.
+// sums of larger ones end in a whole zero or far above) are computed again so.
+//
+// A wave makes an output or four at a time, its lanes side by side along K. Measured (us,
+// plain / one infinite row / all x near 1e-30; with a lane per output before): BF16
+// N 14336 K 4096 M 200 147 / 388 / 2590 (1080 / 30450), N 4096 M 12 21 / 65 / 175 (414 /
+// 768), Q5_K M 200 197 / 598 / 3940 (3290 / 226800), N 4096 M 12 30 / 151 / 361 (1540 / 5470).
+// The GEMVs: 33 and 1560, 70 and 2650.
 template <uint32_t T>
-__device__ __forceinline__ float plain_dot(const FactArgs& g, int m, int n) {
-    const float* x = g.x + (size_t)m * g.K;
-    const uint8_t* w = g.w + (size_t)n * g.rb;
-    float s = 0.0f, sm = 0.0f;            // the mins' sum apart, as the reference keeps it
-    for (int k = 0; k < g.K && s == s; k++) {
-        float mn = 0.0f;
-        if constexpr (T == T_Q2_K) {
-            const uint8_t* b = w + (k >> 8) * 84;
-            mn = fp16_bits_to_f32(rd16(b + 82)) * (float)(b[(k & 255) >> 4] >> 4);
-        } else if constexpr (T == T_Q5_K) {
-            const uint8_t* b = w + (k >> 8) * 176;
-            int sc, mi;
-            scale_min((k & 255) >> 5, b + 4, sc, mi);
-            mn = fp16_bits_to_f32(rd16(b + 2)) * (float)mi;
+__device__ __forceinline__ void decode8(const uint8_t* w, int k, float (&v)[8], float& mn) {
+    mn = 0.0f;
+    if constexpr (T == T_F32) {
+        const u32x4 a = *reinterpret_cast<const u32x4_a4*>(w + 4l * k), b = *reinterpret_cast<const u32x4_a4*>(w + 4l * k + 16);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __uint_as_float(a[i]), v[4 + i] = __uint_as_float(b[i]);
+    } else if constexpr (T == T_F16 || T == T_BF16) {
+        const u32x4 a = *reinterpret_cast<const u32x4_a2*>(w + 2l * k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[2 * i] = T == T_F16 ? fp16_bits_to_f32(a[i]) : lo_f32(a[i]);
+            v[2 * i + 1] = T == T_F16 ? fp16_bits_to_f32(a[i] >> 16) : hi_f32(a[i]);
         }
-        s = fmaf(x[k], dequant_one(T, w, k) + mn, s);
-        if constexpr (Traits<T>::kMin) sm = fmaf(x[k], mn, sm);
+    } else {
+        // 8 values of one 16-element group: their low bits' and high bits' bytes
+        const int e = k & 255, j = e >> 4, g = e >> 5;
+        u32x2 q, h = {0, 0};
+        float d;
+        int sh, hs = 0;
+        if constexpr (T == T_Q2_K) {
+            const uint8_t* b = w + (k >> 8) * 84l;
+            d = fp16_bits_to_f32(rd16(b + 80)) * (float)(b[j] & 15);
+            mn = fp16_bits_to_f32(rd16(b + 82)) * (float)(b[j] >> 4);
+            q = *reinterpret_cast<const u32x2_a2*>(b + 16 + 32 * (g >> 2) + (e & 31));
+            sh = 2 * (g & 3);
+        } else if constexpr (T == T_Q3_K) {
+            const uint8_t* b = w + (k >> 8) * 110l;
+            d = fp16_bits_to_f32(rd16(b + 108)) * (float)(q3k_scale(b + 96, j) - 32);
+            q = *reinterpret_cast<const u32x2_a2*>(b + 32 + 32 * (g >> 2) + (e & 31));
+            h = *reinterpret_cast<const u32x2_a2*>(b + (e & 31));
+            sh = 2 * (g & 3);
+            hs = g;
+        } else {
+            const uint8_t* b = w + (k >> 8) * 176l;
+            int sc, mi;
+            scale_min(g, b + 4, sc, mi);
+            d = fp16_bits_to_f32(rd16(b)) * (float)sc;
+            mn = fp16_bits_to_f32(rd16(b + 2)) * (float)mi;
+            q = *reinterpret_cast<const u32x2_a2*>(b + 48 + 32 * (g >> 1) + (e & 31));
+            h = *reinterpret_cast<const u32x2_a2*>(b + 16 + (e & 31));
+            sh = 4 * (g & 1);
+            hs = g;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t lo = (q[i >> 2] >> (8 * (i & 3) + sh)) & (T == T_Q5_K ? 15u : 3u), hi = (h[i >> 2] >> (8 * (i & 3) + hs)) & 1u;
+            v[i] = d * (T == T_Q3_K ? (float)((int)(lo + 4 * hi) - 4) : (float)(T == T_Q5_K ? lo + 16 * hi : lo));
+        }
     }
-    return s - sm;
+}
+// R rows of x from m0 on (those past M: the last one) times column n, the sums of type S in
+// every lane; the mins' sums apart, as the reference keeps them
+template <uint32_t T, int R, typename S>
+__device__ __forceinline__ void wave_dot(const FactArgs& g, int m0, int n, int lane, float (&out)[R]) {
+    const uint8_t* w = g.w + (size_t)n * g.rb;
+    S s[R] = {}, sm[R] = {};
+#pragma unroll R == 1 ? 4 : 2
+    for (int k = 8 * lane; k < g.K; k += 512) {
+        float v[8], mn;
+        decode8<T>(w, k, v, mn);
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            const float* x = g.x + (size_t)(m0 + i < g.M ? m0 + i : g.M - 1) * g.K + k;
+            const float4 a = *reinterpret_cast<const float4*>(x), b = *reinterpret_cast<const float4*>(x + 4);
+            const float u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int l = 0; l < 8; l++) {
+                s[i] = __builtin_elementwise_fma((S)u[l], (S)v[l], s[i]);
+                if constexpr (Traits<T>::kMin) sm[i] = __builtin_elementwise_fma((S)u[l], (S)mn, sm[i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; i++) out[i] = (float)(Traits<T>::kMin ? wave_sum(s[i]) - wave_sum(sm[i]) : wave_sum(s[i]));
 }
 __device__ __forceinline__ bool suspect(float v) {
     const uint32_t e = (__float_as_uint(v) >> 23) & 0xffu;
     return e == 255u || (e < 127u - 80u && v != 0.0f);
+}
+
+// LDS of the stages, and after them of the K groups' sums
+template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
+constexpr int lds_bytes() {
+    constexpr int red = WK > 1 ? WK * WM * WN * MT * NT * 8192 : 0;
+    constexpr int bufs = WK * (WM * WN == 1 ? 1 : 2) * Lay<T, 32 * MT * WM, 32 * NT * WN>::bytes;
+    return bufs > red ? bufs : red;
 }
 
 // MT x NT tiles of 32 x 32 per wave.
@@ -285,6 +353,8 @@ gemm_fact(FactArgs g) {
     // a group of one wave needs no barrier and one buffer: its LDS operations are in order
     constexpr int NBUF = GT == 64 ? 1 : 2;
     uint8_t* const lds = smem + kg * NBUF * L::bytes;
+    uint32_t* const again = reinterpret_cast<uint32_t*>(smem + lds_bytes<T, MT, NT, WM, WN, WK>());
+    if (threadIdx.x == 0) *again = 0;      // whether the tile has outputs to make again
 
     // tile order: as in the int8 product (one near-square block of tiles per XCD)
     const int ntiles = g.ntm * g.ntn, bid = blockIdx.x;
@@ -487,12 +557,23 @@ gemm_fact(FactArgs g) {
         else __syncthreads();
     }
 
+    // register j = (t * NT + r) * 16 + i of a lane: its token and weight row (the lane's
+    // number is read again, so that the part below keeps no register through the loop)
+    const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    auto mrow = [&](int j) { return m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * ((j & 15) >> 2) + 4 * (ln >> 5) + (j & 3); };
+    auto nrow = [&](int j) { return n0 + (wn * NT + (j >> 4) % NT) * 32 + (ln & 31); };
+    bool bad = false;
+    auto put = [&](int j, float v) {
+        const int m = mrow(j), n = nrow(j);
+        if (m < g.M && n < g.N) g.y[(size_t)m * g.N + n] = v;
+        bad |= suspect(v);
+    };
     if constexpr (WK > 1) {
         __syncthreads();      // every wave is done with its buffer
         // All groups leave their sums in LDS; group kg adds those of registers kg,
         // kg + WK, .. in the groups' order (against one group adding the others' one
         // after the other: BF16 N 4096 K 4096 M 12 21.4 -> 19.6 us).
-        double* red = reinterpret_cast<double*>(smem) + wave * MT * NT * 16 * 64 + lane;
+        double* red = reinterpret_cast<double*>(smem) + wave * MT * NT * 16 * 64 + ln;
         constexpr int kGrp = WM * WN * MT * NT * 16 * 64;
 #pragma unroll
         for (int t = 0; t < MT; t++)
@@ -505,44 +586,72 @@ gemm_fact(FactArgs g) {
             double u = red[j * 64];
 #pragma unroll
             for (int q = 1; q < WK; q++) u += red[q * kGrp + j * 64];
-            const int i = j & 15, n = n0 + (wn * NT + (j >> 4) % NT) * 32 + col;
-            const int m = m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-            if (m < g.M && n < g.N) {
-                const float v = (float)u;
-                g.y[(size_t)m * g.N + n] = suspect(v) ? plain_dot<T>(g, m, n) : v;
-            }
+            put(j, (float)u);
         }
-        return;
-    }
-    bool bad = false;
-#pragma unroll
-    for (int r = 0; r < NT; r++) {
-        const int n = n0 + (wn * NT + r) * 32 + col;
+    } else {
 #pragma unroll
         for (int t = 0; t < MT; t++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int m = m0 + (wm * MT + t) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (m < g.M && n < g.N) g.y[(size_t)m * g.N + n] = (float)sum[t][r][i];
-                bad |= suspect((float)sum[t][r][i]);
-            }
+            for (int r = 0; r < NT; r++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) put((t * NT + r) * 16 + i, (float)sum[t][r][i]);
     }
-    if (!__any(bad)) return;
-    for (int j = 0; j < MT * NT * 16; j++) {
-        const int i = j & 15, n = n0 + (wn * NT + (j >> 4) / MT) * 32 + col;
-        const int m = m0 + (wm * MT + (j >> 4) % MT) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-        if (m >= g.M || n >= g.N) continue;
-        float* y = g.y + (size_t)m * g.N + n;
-        if (suspect(*y)) *y = plain_dot<T>(g, m, n);
+    if (bad) *again = 1;
+    __syncthreads();
+    if (__builtin_expect(*again == 0, 1)) return;
+
+    // units of four registers, i.e. of four rows in a column
+    for (int u = kg; u < MT * NT * 4; u += WK) {
+        const int m = mrow(4 * u), n = nrow(4 * u);
+        float* const y = g.y + (size_t)m * g.N + n;
+        uint32_t todo = 0, nans = 0, inf = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (m + i >= g.M || n >= g.N) continue;
+            const float v = y[(size_t)i * g.N];
+            if (suspect(v)) todo |= 1u << i;
+            if (v != v) nans |= 1u << i;
+            if (!(fabsf(v) < __builtin_inff())) inf |= 1u << i;
+        }
+        // a NaN in x makes its row NaN: nothing to be made again
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint64_t b = __ballot((nans >> (i & 3)) & 1u) & (i < 4 ? 0xffffffffull : ~0xffffffffull);
+            if (!b) continue;
+            const float* x = g.x + (size_t)(__builtin_amdgcn_readlane(m, i < 4 ? 0 : 32) + (i & 3)) * g.K;
+            bool nan = false;
+            for (int k = 4 * ln; k < g.K && !__any(nan); k += 256) {
+                const float4 a = *reinterpret_cast<const float4*>(x + k);
+                nan = a.x != a.x || a.y != a.y || a.z != a.z || a.w != a.w;
+            }
+            if (__any(nan) && (ln >> 5) == (i >> 2)) todo &= ~(1u << (i & 3));
+        }
+        // non-finite ones singly in 64 bits (a lane's share may leave the fp32 range where
+        // the sum does not), small ones of the four rows at once
+        for (uint64_t left = __ballot(todo != 0); left; left &= left - 1) {
+            const int l = __ffsll((unsigned long long)left) - 1;
+            const int ml = __builtin_amdgcn_readlane(m, l), nl = __builtin_amdgcn_readlane(n, l);
+            const uint32_t td = __builtin_amdgcn_readlane(todo, l), large = __builtin_amdgcn_readlane(inf, l) & td;
+            for (int i = 0; i < 4; i++) {
+                if (!((large >> i) & 1u)) continue;
+                float v[1];
+                wave_dot<T, 1, double>(g, ml + i, nl, ln, v);
+                if (ln == l) y[(size_t)i * g.N] = v[0];
+            }
+            if (td == large) continue;
+            float v[4];
+            wave_dot<T, 4, float>(g, ml, nl, ln, v);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (ln == l && (((td ^ large) >> i) & 1u)) y[(size_t)i * g.N] = v[i];
+        }
     }
 }
 
 template <uint32_t T, int MT, int NT, int WM, int WN, int WK>
 hipError_t launch_cfg(FactArgs g, hipStream_t st) {
     constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
-    constexpr int red = WK > 1 ? WK * WM * WN * MT * NT * 8192 : 0;
-    constexpr int bufs = WK * (WM * WN == 1 ? 1 : 2) * Lay<T, BM, BN>::bytes;
-    constexpr int lds = bufs > red ? bufs : red;
+    constexpr int lds = lds_bytes<T, MT, NT, WM, WN, WK>() + 16;            // and a flag
     static_assert(lds <= 160 * 1024, "LDS");
     g.ntm = (g.M + BM - 1) / BM;
     g.ntn = (g.N + BN - 1) / BN;
