@@ -75,11 +75,20 @@ __device__ __forceinline__ float lo_f32(uint32_t p) { return __uint_as_float(p <
 __device__ __forceinline__ float hi_f32(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 __device__ __forceinline__ float hi16(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
 
+// What a thread has met of the values whose pieces do not hold all their bits: the x
+// tasks (a bit each) with a quadruple below 2^-100 that is not all zeros; F32 only: the
+// largest finite magnitude from 2^20 up, and the x and w tasks with such values.
+struct Ends {
+    uint32_t tiny = 0, xbig = 0, wbig = 0;
+    float big = 0.0f;
+};
+
 // v[4] as PL planes of 4 bf16 whose sum is v: each piece is the rest rounded to
 // nearest. Values whose first piece would round to infinity, and infinities
-// (their own first piece), are cut off instead.
-template <int PL>
-__device__ __forceinline__ void split4(const float (&v)[4], u32x2 (&o)[PL]) {
+// (their own first piece), are cut off instead. One comparison finds these and the
+// quadruples that Ends counts (all zeros among them).
+template <int PL, bool BIG, bool X>
+__device__ __forceinline__ void split4(const float (&v)[4], u32x2 (&o)[PL], Ends& e, uint32_t bit) {
     float r[4];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -90,7 +99,18 @@ __device__ __forceinline__ void split4(const float (&v)[4], u32x2 (&o)[PL]) {
         if constexpr (PL > 2)
             o[2][i] = pk_bf16(r[2 * i] - lo_f32(o[1][i]), r[2 * i + 1] - hi_f32(o[1][i]));
     }
-    if (PL > 1 && fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))) >= 0x1.fe8p127f) {
+    if constexpr (PL == 1) return;
+    const float a = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    constexpr float top = BIG ? 0x1p20f : 0x1.fe8p127f;
+    constexpr uint32_t lo = X ? (127u - 100u) << 23 : 0u;
+    if (__builtin_expect(__float_as_uint(a) - lo < __builtin_bit_cast(uint32_t, top) - lo, 1)) return;
+    if (BIG && a >= top) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) e.big = fmaxf(e.big, fabsf(v[i]) < __builtin_inff() ? fabsf(v[i]) : 0.0f);
+        (X ? e.xbig : e.wbig) |= bit;
+    }
+    if (X && a > 0.0f && a < 0x1p-100f) e.tiny |= bit;
+    if (a >= 0x1.fe8p127f) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             uint32_t q[2][3];
@@ -160,7 +180,7 @@ struct Lay {
 };
 
 template <uint32_t T, int BM, int BN>
-__device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, int s, int t, bool on) {
+__device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, int s, int t, bool on, Ends& ends, uint32_t bit) {
     typedef Lay<T, BM, BN> L;
     constexpr int PL = Traits<T>::kPlanes;
     uint8_t* wt = st + L::w + (n >> 5) * kTile + (n & 31) * 16;
@@ -178,7 +198,7 @@ __device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, in
                 v[i] = on ? v[i] : 0.0f;
             }
             u32x2 o[PL];
-            split4<PL>(v, o);
+            split4<PL, T == T_F32, false>(v, o, ends, bit);
             uint8_t* p = T == T_F32 ? wt + (t >> 1) * kH + 8 * (t & 1) : wt + t * kH + 8 * h;
 #pragma unroll
             for (int k = 0; k < PL; k++) *reinterpret_cast<u32x2*>(p + k * (BN / 32) * kTile) = o[k];
@@ -235,12 +255,23 @@ __device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, in
     }
 }
 
-// Outputs made again in fp32. The pieces of an infinity are (inf, 0, 0) and its product
-// with a zero piece of a finite value is NaN, so are partial sums past the fp32
-// range with opposite signs, and the matrix unit takes pieces below 2^-126 as zero
-// (third pieces of values below 2^-108). Outputs that come out infinite, NaN or
-// nonzero and below 2^-80 (there by such values, not by cancellation: the 64-bit
-// sums of larger ones end in a whole zero or far above) are computed again so.
+// Outputs that the pieces do not give are made again in fp32:
+//  - infinite and NaN ones: the pieces of an infinity are (inf, 0, 0) and its product
+//    with a zero piece of a finite value is NaN, so are partial sums past the fp32
+//    range with opposite signs;
+//  - those that bits below the pieces' last one could show in: bf16 ends at 2^-133
+//    (the matrix unit keeps such denormals, and its fp32 results'), so the pieces of
+//    an x are off by up to 2^-134 where it is below 2^-110, and the sum by up to
+//    K 2^-134 times the largest weight: 2^16 in F16, below 2^28 in the quantized types
+//    and 2^20 in F32 and BF16, or what was met in an F32 column beyond that. (F32 weights
+//    have the same pieces beside the largest x of the row.) Outputs below K 2^-110 times
+//    that size are suspect; ordinary sums do not come there by cancellation, their 64-bit
+//    sums end in a whole zero or far above;
+//  - the rows of x with four neighbours all below 2^-100, not all zero: BF16 weights are not
+//    looked at on their way to LDS and may be of any size.
+// What is left: a sum of values below 2^-134 among larger ones may come out 0, and of BF16
+// weights beyond 2^20 those beside an x below 2^-110 whose three neighbours are larger count
+// with its first bits.
 //
 // A wave makes an output or four at a time, its lanes side by side along K. Measured (us,
 // plain / one infinite row / all x near 1e-30; with a lane per output before): BF16
@@ -323,9 +354,9 @@ __device__ __forceinline__ void wave_dot(const FactArgs& g, int m0, int n, int l
 #pragma unroll
     for (int i = 0; i < R; i++) out[i] = (float)(Traits<T>::kMin ? wave_sum(s[i]) - wave_sum(sm[i]) : wave_sum(s[i]));
 }
-__device__ __forceinline__ bool suspect(float v) {
-    const uint32_t e = (__float_as_uint(v) >> 23) & 0xffu;
-    return e == 255u || (e < 127u - 80u && v != 0.0f);
+__device__ __forceinline__ bool suspect(float v, float below) {
+    const float a = fabsf(v);
+    return !(a == 0.0f || (a >= below && a < __builtin_inff()));
 }
 
 // LDS of the stages, and after them of the K groups' sums
@@ -355,6 +386,7 @@ gemm_fact(FactArgs g) {
     uint8_t* const lds = smem + kg * NBUF * L::bytes;
     uint32_t* const again = reinterpret_cast<uint32_t*>(smem + lds_bytes<T, MT, NT, WM, WN, WK>());
     if (threadIdx.x == 0) *again = 0;      // whether the tile has outputs to make again
+    Ends ends;
 
     // tile order: as in the int8 product (one near-square block of tiles per XCD)
     const int ntiles = g.ntm * g.ntn, bid = blockIdx.x;
@@ -401,7 +433,7 @@ gemm_fact(FactArgs g) {
             const int row = (tid + i * GT) >> 4;
             const float v[4] = {on ? rx[i].x : 0.0f, on ? rx[i].y : 0.0f, on ? rx[i].z : 0.0f, on ? rx[i].w : 0.0f};
             u32x2 o[3];
-            split4<3>(v, o);
+            split4<3, T == T_F32, true>(v, o, ends, 1u << i);
             uint8_t* p = st + L::x + (row >> 5) * kTile + (quad >> 1) * kH + (row & 31) * 16 + 8 * (quad & 1);
 #pragma unroll
             for (int k = 0; k < 3; k++) *reinterpret_cast<u32x2*>(p + k * (BM / 32) * kTile) = o[k];
@@ -428,7 +460,7 @@ gemm_fact(FactArgs g) {
         for (int i = 0; i < WPT; i++) {
             const int p = tid + i * GT, t = p % R::kTasks;
             if (BN * R::kTasks % GT == 0 || p < BN * R::kTasks)
-                w_store<T, BM, BN>(rw[i], st, p / R::kTasks, sw, t, 64 * s + (R::kQuant ? 0 : 64 / R::kTasks * t) < g.K);
+                w_store<T, BM, BN>(rw[i], st, p / R::kTasks, sw, t, 64 * s + (R::kQuant ? 0 : 64 / R::kTasks * t) < g.K, ends, 1u << i);
         }
     };
 
@@ -562,11 +594,13 @@ gemm_fact(FactArgs g) {
     const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     auto mrow = [&](int j) { return m0 + (wm * MT + (j >> 4) / NT) * 32 + 8 * ((j & 15) >> 2) + 4 * (ln >> 5) + (j & 3); };
     auto nrow = [&](int j) { return n0 + (wn * NT + (j >> 4) % NT) * 32 + (ln & 31); };
+    constexpr float kSize = T == T_F16 ? 0x1p16f : R::kQuant ? 0x1p28f : 0x1p20f;
+    const float below = (float)g.K * (0x1p-110f * kSize);
     bool bad = false;
     auto put = [&](int j, float v) {
         const int m = mrow(j), n = nrow(j);
         if (m < g.M && n < g.N) g.y[(size_t)m * g.N + n] = v;
-        bad |= suspect(v);
+        bad |= suspect(v, below);
     };
     if constexpr (WK > 1) {
         __syncthreads();      // every wave is done with its buffer
@@ -596,10 +630,22 @@ gemm_fact(FactArgs g) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) put((t * NT + r) * 16 + i, (float)sum[t][r][i]);
     }
-    if (bad) *again = 1;
+    if (bad || ends.tiny || ends.big > 0.0f) *again = 1;
     __syncthreads();
     if (__builtin_expect(*again == 0, 1)) return;
 
+    // of the tile's x and weight rows: the largest magnitude from 2^20 up, all bits set for tiny x rows
+    uint32_t* const ex = reinterpret_cast<uint32_t*>(smem);
+    const int tg = (int)(threadIdx.x % GT);
+    for (int i = threadIdx.x; i < BM + BN; i += GT * WK) ex[i] = 0;
+    __syncthreads();
+    for (int i = 0; i < XPT; i++) {
+        const uint32_t v = (ends.tiny >> i) & 1u ? ~0u : (ends.xbig >> i) & 1u ? __float_as_uint(ends.big) : 0u;
+        if (v) atomicMax(ex + ((tg + i * GT) >> 4), v);
+    }
+    for (int i = 0; i < WPT; i++)
+        if ((ends.wbig >> i) & 1u) atomicMax(ex + BM + (tg + i * GT) / R::kTasks, __float_as_uint(ends.big));
+    __syncthreads();
     // units of four registers, i.e. of four rows in a column
     for (int u = kg; u < MT * NT * 4; u += WK) {
         const int m = mrow(4 * u), n = nrow(4 * u);
@@ -609,7 +655,9 @@ gemm_fact(FactArgs g) {
         for (int i = 0; i < 4; i++) {
             if (m + i >= g.M || n >= g.N) continue;
             const float v = y[(size_t)i * g.N];
-            if (suspect(v)) todo |= 1u << i;
+            const uint32_t xe = ex[m + i - m0], we = ex[BM + n - n0];
+            const float size = fmaxf(kSize, __uint_as_float(xe > we ? xe : we));
+            if (xe == ~0u || suspect(v, (float)g.K * 0x1p-110f * size)) todo |= 1u << i;
             if (v != v) nans |= 1u << i;
             if (!(fabsf(v) < __builtin_inff())) inf |= 1u << i;
         }

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from hip_util import normwise
-from test_gpu_fact import BF16, F16, F32, FACT, Q2_K, Q3_K, Q5_K, fact_weights, gemm_dev
+from test_gpu_fact import BF16, BLOCK, F16, F32, FACT, Q2_K, Q3_K, Q5_K, fact_weights, gemm_dev
 
 pytestmark = pytest.mark.gpu
 DENSE = {"F32": F32, "F16": F16, "BF16": BF16}
@@ -150,6 +150,60 @@ def test_fact_gemm_line(name):
         y = gemm_dev(t, x, w, N)
         for part in (gemm_dev(t, x[:m0 - 1], w, N), gemm_dev(t, x[:2], w, N)):
             assert normwise(y[:len(part)], part) <= TOL
+
+
+# powers of two of x and of the weights: x (or w) with pieces below 2^-126 beside factors
+# that bring the products back to ordinary size, and products near the ends of the range
+RANGES = [(-118, 40), (-130, 60), (-145, 100), (-112, 20), (40, -118), (90, -131), (-70, -70), (-60, -62), (100, -100), (-40, 0)]
+
+
+@pytest.mark.parametrize("ex,ew", RANGES)
+@pytest.mark.parametrize("name", list(DENSE))
+@pytest.mark.parametrize("M,N", [(40, 2500), (64, 14400), (200, 24600)])
+def test_fact_gemm_operand_ranges(name, M, N, ex, ew):
+    """Tiny values against large ones keep the bits that fp32 products keep, on either
+    side; rows and columns of ordinary size beside them keep theirs."""
+    t = DENSE[name]
+    if t == F16 and not -24 <= ew <= 14:
+        pytest.skip("outside fp16")
+    K = 96
+    rng = np.random.default_rng(200 + ex + 1000 * (200 + ew))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    v = rng.standard_normal((N, K)).astype(np.float32)
+    x[1], x[M - 1] = x[1] * 2.0 ** ex, 0
+    x[3, ::5] *= np.float32(2.0 ** ex)
+    x[M - 1, 70] = 1.375 * 2.0 ** ex
+    v[5], v[N - 1] = v[5] * 2.0 ** ew, v[N - 1] * 2.0 ** ew
+    v[6, ::5] *= np.float32(2.0 ** ew)
+    v, wb = dense(t, v)
+    y = gemm_dev(t, x, wb, N)
+    cols = [0, 5, 6, N // 2, N - 1]
+    p = x.astype(np.float64)[:, None] * v.astype(np.float64)[None, cols]
+    ref, size = p.sum(-1), np.abs(p).sum(-1)
+    # the fp32 dots' own error: at most K roundings of partial sums, denormal ones absolute
+    bad = np.abs(y[:, cols] - ref) > 2.0 ** -21 * size + K * 2.0 ** -149
+    assert not bad.any(), np.argwhere(bad)[:8]
+
+
+@pytest.mark.parametrize("name", ["Q2_K", "Q3_K", "Q5_K"])
+def test_fact_gemm_tiny_rows_large_scales(name):
+    """Rows near 2^-112 with the largest block scales are the ordinary rows' products, scaled:
+    the outputs lie near 2^-90."""
+    t = FACT[name]
+    M, N, K = 40, 2500, 512
+    w = fact_weights(t, K, N, seed=7)
+    _, size, at = BLOCK[t]
+    for o in at:
+        w.reshape(-1, size)[:, o:o + 2] = np.array([6e4], np.float16).view(np.uint8)
+    x = np.random.default_rng(9).standard_normal((M, K)).astype(np.float32)
+    plain = gemm_dev(t, x, w, N)
+    z = x.copy()
+    z[::3] *= np.float32(2.0 ** -112)
+    y = gemm_dev(t, z, w, N)
+    for m in range(0, M, 3):
+        assert normwise(y[m] * np.float32(2.0 ** 112), plain[m]) <= TOL
+    rest = [m for m in range(M) if m % 3]
+    assert np.array_equal(y[rest].view(np.uint32), plain[rest].view(np.uint32))
 
 
 @pytest.mark.parametrize("M,N", [(12, 8190), (200, 2500)])
