@@ -966,7 +966,7 @@ gemv_q4k_i8mf(const uint8_t* __restrict__ w, long rb, ActView A, float* __restri
     }
 }
 
-// Q6_K for 5 <= M <= 16 on the same int8 MFMA: B = the 6-bit codes minus 32
+// Q6_K for 9 <= M <= 16 on the same int8 MFMA: B = the 6-bit codes minus 32
 // as int8 (ql nibble | qh bits << 4, then -32 per byte), so D is the exact
 // sum of (code - 32) * q. The two 16-element halves of a 32-element block
 // have their own int8 scale, so a block takes two MFMAs (lanes of the other
@@ -1106,17 +1106,11 @@ hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, f
     if (q6rq_preferred(type, M, K, N, w)) return launch_gemv_q6rq(w, A, y, M, K, N, st);
     const dim3 grid((N + 16 * kMfTiles - 1) / (16 * kMfTiles));
     if (type == T_Q6_K) {
-        // few weight rows (e.g. a down projection, 3584 rows of K 18944): 16-row
-        // workgroups of 16 waves, so the K-slices spread over twice the CUs.
-        // Switch point measured for Q6_K and Q8_0, M 8..16: 14336 rows (448
-        // 32-row workgroups) 10-13 % faster on the 32-row form, 10240 rows
-        // (320) 10-13 % faster on the 16-row form.
+        // 9..16 rows, and few weight rows (more than a 32-row tile per CU are the tiled
+        // product's): 16-row workgroups of 16 waves spread the K-slices over the CUs
         const size_t shm = (size_t)(K / 32) * 16 * 4;
         const long rbq = (long)row_bytes(T_Q6_K, K);
-        if (2 * ((N + 31) / 32) >= 3 * device_cu_count())
-            hipLaunchKernelGGL((gemv_q6k_i8mf<2, 8>), grid, dim3(512), shm, st, w, rbq, A, y, M, K, N);
-        else
-            hipLaunchKernelGGL((gemv_q6k_i8mf<1, 16>), dim3((N + 15) / 16), dim3(1024), shm, st, w, rbq, A, y, M, K, N);
+        hipLaunchKernelGGL((gemv_q6k_i8mf<1, 16>), dim3((N + 15) / 16), dim3(1024), shm, st, w, rbq, A, y, M, K, N);
     } else {
         const size_t shm = (size_t)(K / 32) * 16 * 8;
         const long rbq = (long)row_bytes(T_Q4_K, K);

@@ -720,32 +720,43 @@ namespace {
 //         M 2048 (512 tiles of 128 x 128) 128x128 253, 64x64 343
 //   F32   M 128  32x32x6 85, 64x64 119      M 256  64x64 119, 64x128 165
 //         M 512  64x128 169, 64x64 225
-enum Form { F32X32X8, F32X32X4, F64X64X2, F64X64, F64X128, F128X128 };
+// Several planes leave LDS for six K groups of 32 x 32 and for 64 x 128 at most.
+enum Form { F32X32X8, F32X32X6, F32X32X4, F64X64X2, F64X64, F64X128, F128X128 };
 
 template <uint32_t T>
 Form pick_form(int M, int N) {
     const long cus = device_cu_count();
     auto tiles = [&](int b) { return (long)((M + b - 1) / b) * ((N + b - 1) / b); };
     constexpr bool one = Traits<T>::kPlanes == 1;
+    if (!one) return tiles(32) <= 2 * cus || M <= 32 ? F32X32X6 : tiles(64) <= cus ? F64X64 : F64X128;
     if (tiles(32) <= cus) return F32X32X8;
-    if (tiles(32) <= 2 * cus || M <= 32) return one ? F32X32X4 : F32X32X8;
-    if (tiles(64) <= cus) return one ? F64X64X2 : F64X64;
-    if (!one) return F64X128;
+    if (tiles(32) <= 2 * cus || M <= 32) return F32X32X4;
+    if (tiles(64) <= cus) return F64X64X2;
     const long r64 = (tiles(64) + 2 * cus - 1) / (2 * cus), r128 = (tiles(128) + cus - 1) / cus;
     return 1.4 * r128 < r64 ? F128X128 : F64X64;
 }
 
 template <uint32_t T>
 hipError_t launch_t(const FactArgs& g, hipStream_t st) {
-    constexpr bool one = Traits<T>::kPlanes == 1;
-    switch (pick_form<T>(g.M, g.N)) {
-        case F32X32X8: return launch_cfg<T, 1, 1, 1, 1, one ? 8 : 6>(g, st);
-        case F32X32X4: return launch_cfg<T, 1, 1, 1, 1, one ? 4 : 6>(g, st);
-        case F64X64X2: return launch_cfg<T, 1, 1, 2, 2, one ? 2 : 1>(g, st);
-        case F64X64: return launch_cfg<T, 1, 1, 2, 2, 1>(g, st);
-        case F64X128: if constexpr (!one) return launch_cfg<T, 1, 2, 2, 2, 1>(g, st); [[fallthrough]];
-        default: return launch_cfg<T, 1, 2, one ? 4 : 2, 2, 1>(g, st);
+    const Form f = pick_form<T>(g.M, g.N);
+    if constexpr (Traits<T>::kPlanes == 1) {
+        switch (f) {
+            case F32X32X8: return launch_cfg<T, 1, 1, 1, 1, 8>(g, st);
+            case F32X32X4: return launch_cfg<T, 1, 1, 1, 1, 4>(g, st);
+            case F64X64X2: return launch_cfg<T, 1, 1, 2, 2, 2>(g, st);
+            case F64X64: return launch_cfg<T, 1, 1, 2, 2, 1>(g, st);
+            case F128X128: return launch_cfg<T, 1, 2, 4, 2, 1>(g, st);
+            default: break;
+        }
+    } else {
+        switch (f) {
+            case F32X32X6: return launch_cfg<T, 1, 1, 1, 1, 6>(g, st);
+            case F64X64: return launch_cfg<T, 1, 1, 2, 2, 1>(g, st);
+            case F64X128: return launch_cfg<T, 1, 2, 2, 2, 1>(g, st);
+            default: break;
+        }
     }
+    return hipErrorInvalidValue;
 }
 }  // namespace
 

@@ -221,7 +221,7 @@ struct Lay {
 };
 
 template <uint32_t T, int BM, int BN>
-__device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, int b0, int nb, int task) {
+__device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, int b0, int task) {
     typedef Lay<T, BM, BN> L;
     uint8_t* wt = st + L::w + (n >> 5) * kTileBytes + (n & 31) * 16;
     u32x2* wd = reinterpret_cast<u32x2*>(st + L::wd);
@@ -462,7 +462,7 @@ gemm_i8t(I8tArgs g) {
         for (int i = 0; i < WPT; i++) {
             const int p = tid + i * GT;
             if (BN * R::kTasks % GT == 0 || p < BN * R::kTasks)
-                w_store<T, BM, BN>(rw[i], st, p / R::kTasks, b0, nb, p % R::kTasks);
+                w_store<T, BM, BN>(rw[i], st, p / R::kTasks, b0, p % R::kTasks);
         }
     };
 
@@ -846,8 +846,10 @@ hipError_t launch_moe_t(const I8tArgs& g, int gsize, hipStream_t st) {
     switch (gsize) {
         case 32: return launch_cfg<T, 1, 1, 1, 4, 1, true>(g, st);
         case 64: return launch_cfg<T, 1, 1, 2, 2, 1, true>(g, st);
-        case 128: return launch_cfg<T, 2, 1, 2, 4, 1, true>(g, st);
     }
+    // (Q8_0 and Q4_0 stay at 64: moe_i8t_group)
+    if constexpr (T == T_Q4_K || T == T_Q6_K)
+        if (gsize == 128) return launch_cfg<T, 2, 1, 2, 4, 1, true>(g, st);
     return hipErrorInvalidValue;
 }
 }  // namespace
