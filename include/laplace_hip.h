@@ -246,6 +246,17 @@ int lp_set_gemm_kernel(int kernel);
  * it to show which kernel a parity case exercised. */
 const char* lp_gemm_route(uint32_t type, int M, int K, int N, const void* w);
 
+/* The same with the tiled products named apart, for lp_gemm_dev's prompt rows:
+ * "i8t 64x64" (the tiled int8 product) or "fact_gemm 64x64" (the tiled product of
+ * fp32 activations), each with the tile's tokens x weight rows, and "x8" where
+ * that many groups of waves share K; for every other call lp_gemm_route's name. */
+const char* lp_gemm_form(uint32_t type, int M, int K, int N, const void* w);
+
+/* Probe of the grouped MoE dispatch: how many pairs of an expert one group holds
+ * for lp_moe_grouped_dev's arguments (32 and more: the tiled int8 product, 8: the
+ * row-quad kernel, 4: the GEMV kernels); 0 where the call is refused. */
+int lp_moe_group_pairs(uint32_t type, int T, int topk, int n_experts, int K, int multi);
+
 /* Measurement hook, no reference counterpart: streams `bytes` (a multiple
  * of 16) from device memory with `grid` x `block` threads and `unroll`
  * (1, 4 or 9) independent 16-byte non-temporal loads in flight per thread,

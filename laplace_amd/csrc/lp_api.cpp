@@ -691,6 +691,19 @@ const char* lp_gemm_route(uint32_t type, int M, int K, int N, const void* w) {
     return gemm_q_route(type, M, K, N, wb);
 }
 
+const char* lp_gemm_form(uint32_t type, int M, int K, int N, const void* w) {
+    const uint8_t* wb = static_cast<const uint8_t*>(w);
+    if (check_shape(type, wb, M, K, N) != LP_OK || M <= 0 || N <= 0) return "";
+    if (fact_type(type)) return fact_gemm_preferred(type, M, K, N) ? fact_gemm_form(type, M, N) : "fact";
+    if (use_i8t(type, M, K, N)) return i8t_form(type, M, N);
+    return gemm_q_route(type, M, K, N, wb);
+}
+
+int lp_moe_group_pairs(uint32_t type, int T, int topk, int n_experts, int K, int multi) {
+    if (check_moe(type, nullptr, T, topk, n_experts, K, 1) != LP_OK) return 0;
+    return moe_group_size(type, multi ? T * topk : T, K, T * topk, n_experts);
+}
+
 int lp_gemm_dev(const float* x, const uint8_t* w, uint32_t type, float* y, int M, int K, int N,
                 void* ws, size_t wsb, void* stream) {
     int rc = check_shape(type, w, M, K, N);

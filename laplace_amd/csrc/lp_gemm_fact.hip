@@ -778,6 +778,19 @@ bool fact_gemm_preferred(uint32_t type, int M, int K, int N) {
     return M >= (type == T_F16 ? 6 : 5) && (long)M * N >= (K <= 2048 ? 2 * line : line);
 }
 
+const char* fact_gemm_form(uint32_t type, int M, int N) {
+    const Form f = type == T_F32 ? pick_form<T_F32>(M, N) : type == T_F16 ? pick_form<T_F16>(M, N) : pick_form<T_BF16>(M, N);
+    switch (f) {
+        case F32X32X8: return "fact_gemm 32x32x8";
+        case F32X32X6: return "fact_gemm 32x32x6";
+        case F32X32X4: return "fact_gemm 32x32x4";
+        case F64X64X2: return "fact_gemm 64x64x2";
+        case F64X64: return "fact_gemm 64x64";
+        case F64X128: return "fact_gemm 64x128";
+        default: return "fact_gemm 128x128";
+    }
+}
+
 hipError_t launch_gemm_fact(uint32_t type, const uint8_t* w, const float* x, float* y, int M, int K, int N,
                             hipStream_t st) {
     if (M <= 0 || N <= 0) return hipSuccess;

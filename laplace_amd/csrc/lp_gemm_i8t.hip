@@ -804,6 +804,16 @@ bool i8t_preferred(uint32_t type, int M, int K, int N) {
     return false;
 }
 
+const char* i8t_form(uint32_t type, int M, int N) {
+    switch (pick_form(type, M, N)) {
+        case F32X32X8: return "i8t 32x32x8";
+        case F32X32X4: return "i8t 32x32x4";
+        case F64X64X2: return "i8t 64x64x2";
+        case F64X64: return "i8t 64x64";
+        default: return "i8t 128x128";
+    }
+}
+
 hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
                            hipStream_t st) {
     if (M <= 0 || N <= 0) return hipSuccess;

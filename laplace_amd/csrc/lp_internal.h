@@ -64,6 +64,7 @@ hipError_t launch_gemv_fact(uint32_t type, const uint8_t* w, const float* x, flo
 // Tiled bf16-MFMA product at fp32 precision for the same types (lp_gemm_fact.hip);
 // launch_gemv_fact takes it where fact_gemm_preferred says so.
 bool fact_gemm_preferred(uint32_t type, int M, int K, int N);
+const char* fact_gemm_form(uint32_t type, int M, int N);      // its tile form (lp_gemm_form)
 hipError_t launch_gemm_fact(uint32_t type, const uint8_t* w, const float* x, float* y, int M, int K, int N,
                             hipStream_t st);
 
@@ -102,6 +103,7 @@ bool i8mf_supported(uint32_t type, int M, int K, int N, const uint8_t* w);
 // Tiled int8 MFMA product of the quantized blocks (lp_gemm_i8t.hip) for all five
 // int8 types; i8t_preferred: the shapes where it is the fastest kernel.
 bool i8t_preferred(uint32_t type, int M, int K, int N);
+const char* i8t_form(uint32_t type, int M, int N);            // its tile form (lp_gemm_form)
 hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
                            hipStream_t st);
 hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,

@@ -38,6 +38,11 @@ def stream():
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def form(t: int, M: int, K: int, N: int) -> str:
+    """The kernel and tile form of lp_gemm_dev for aligned operands."""
+    return L().lp_gemm_form(t, M, K, N, None).decode()
+
+
 def workspace(M: int, K: int):
     torch = torch_dev()
     nb = int(L().lp_act_workspace_bytes(M, K))

@@ -3,7 +3,7 @@ edges of its tiles and forms, against 64-bit products and the oracle."""
 import numpy as np
 import pytest
 
-from hip_util import normwise
+from hip_util import form, normwise
 from test_gpu_fact import BF16, BLOCK, F16, F32, FACT, Q2_K, Q3_K, Q5_K, fact_weights, gemm_dev
 
 pytestmark = pytest.mark.gpu
@@ -17,18 +17,30 @@ TOL = 4e-6
 
 # (M, N, K): one token and one row past a 32- and 64-tile, K ending 32 elements into
 # a 64-element stage (the unquantized types), fewer stages than K groups
-SHAPES = [(33, 3001, 256), (65, 1537, 512), (8, 12289, 768), (127, 449, 2048)]
-TAILS = [(33, 3001, 32), (65, 1537, 96), (8, 12289, 288), (127, 801, 1056)]
+SHAPES = [(33, 3001, 256), (65, 1537, 512), (8, 12289, 2304), (127, 900, 2048)]
+TAILS = [(33, 3001, 32), (65, 1537, 96), (16, 8190, 288), (127, 801, 1056)]
 # M and N that take each form: 32x32 with 8 (6) and 4 K groups, 64x64 with 2 and 1,
-# 64x128, 128x128 (and its edges)
-FORMS = [(31, 8200, 256), (40, 8200, 256), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256)]
+# 64x128, 128x128 (and its edges): test_every_form_is_run
+FORMS = [(31, 8200, 256), (40, 8200, 256), (33, 14400, 256), (70, 8200, 256), (96, 16500, 256), (200, 24600, 256)]
 CASES = [(t, *s) for t in FACT for s in SHAPES + FORMS] + [(t, *s) for t in DENSE for s in TAILS]
+
+
+def test_every_form_is_run():
+    """The cases run each tile form of the product for each type (on 256 CUs)."""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the forms' lines depend on the CU count")
+    for name, t in FACT.items():
+        got = {form(t, M, K, N) for n, M, N, K in CASES if n == name}
+        forms = ("32x32x6", "64x64", "64x128") if name in ("F32", "F16") else ("32x32x8", "32x32x4", "64x64x2", "64x64", "128x128")
+        assert got == {f"fact_gemm {f}" for f in forms}, (name, got)
 
 
 @pytest.mark.parametrize("name,M,N,K", CASES)
 def test_fact_gemm_matches_oracle(orc, name, M, N, K):
     print(f"fact gemm {name} M={M} N={N} K={K}", flush=True)
     t = FACT[name]
+    assert form(t, M, K, N).startswith("fact_gemm ")
     w = fact_weights(t, K, N, seed=M + N + K + t)
     x = np.random.default_rng(M + 1).standard_normal((M, K)).astype(np.float32)
     x[M // 2, :32] = 0.0
@@ -55,6 +67,7 @@ def test_fact_gemm_pieces_keep_fp32(name, scale):
     output leaves its own rounding and the pieces' last bits."""
     t = DENSE[name]
     M, N, K = 64, 1600, 64
+    assert form(t, M, K, N).startswith("fact_gemm ")
     rng = np.random.default_rng(3)
     x = np.zeros((M, K), np.float32)
     x[np.arange(M), np.arange(M)] = ((0.5 + rng.random(M)) * scale).astype(np.float32)
@@ -70,6 +83,7 @@ def test_fact_gemm_quantized_extremes(orc, name):
     match the oracle; the rows beside them stay as they are."""
     t = FACT[name]
     M, N, K = 40, 1700, 512
+    assert form(t, M, K, N).startswith("fact_gemm ")
     w = fact_weights(t, K, N, seed=4)
     x = np.random.default_rng(6).standard_normal((M, K)).astype(np.float32)
     x[1, 7], x[2, 500], x[M - 1, 511] = np.inf, np.nan, -np.inf
@@ -95,6 +109,7 @@ def test_fact_gemm_non_finite(name, M, N):
     t = DENSE[name]
     K = 96
     rng = np.random.default_rng(5)
+    assert form(t, M, K, N).startswith("fact_gemm ")
     x = rng.integers(-4, 5, (M, K)).astype(np.float32)
     v = rng.integers(-4, 5, (N, K)).astype(np.float32)
     x[x == 0] = 1
@@ -123,6 +138,7 @@ def test_fact_gemm_unaligned_weights(name):
     from hip_util import L, stream, to_dev
     t = FACT[name]
     M, N, K = 40, 2500, 96
+    assert form(t, M, K, N).startswith("fact_gemm ")
     w = fact_weights(t, K, N, seed=1)
     x = np.random.default_rng(2).standard_normal((M, K)).astype(np.float32)
     want = gemm_dev(t, x, w, N)
@@ -137,19 +153,17 @@ def test_fact_gemm_unaligned_weights(name):
 
 @pytest.mark.parametrize("name", list(FACT))
 def test_fact_gemm_line(name):
-    """On either side of the line between the GEMVs and this product (24000 outputs,
-    32000 of Q2_K, 49000 in one round of tiles of F16 and F32, twice that up to K = 2048;
-    5 rows, 6 of F16) the rows agree."""
+    """One weight row fewer than the least that takes this product runs on the GEMVs, for
+    the fewest rows, for 16 and at short K (where the line is twice as high): the columns
+    agree."""
     t = FACT[name]
-    line = 49000 if t in (F32, F16) else 32000 if t == Q2_K else 24000
-    m0 = 6 if t == F16 else 5
     rng = np.random.default_rng(8)
-    for M, N, K in ((m0, -(-line // m0), 4096), (16, -(-line // 16), 4096), (16, -(-line // 8), 512)):
+    for M, K in ((6 if name in ("F32", "F16") else 5, 4096), (16, 4096), (16, 512)):
+        N = next(n for n in range(32, 40000) if form(t, M, K, n) != "fact")
         w = fact_weights(t, K, N, seed=N)
         x = rng.standard_normal((M, K)).astype(np.float32)
-        y = gemm_dev(t, x, w, N)
-        for part in (gemm_dev(t, x[:m0 - 1], w, N), gemm_dev(t, x[:2], w, N)):
-            assert normwise(y[:len(part)], part) <= TOL
+        below = gemm_dev(t, x, w[:(N - 1) * (len(w) // N)], N - 1)
+        assert normwise(gemm_dev(t, x, w, N)[:, :-1], below) <= TOL
 
 
 # powers of two of x and of the weights: x (or w) with pieces below 2^-126 beside factors
@@ -167,6 +181,7 @@ def test_fact_gemm_operand_ranges(name, M, N, ex, ew):
     if t == F16 and not -24 <= ew <= 14:
         pytest.skip("outside fp16")
     K = 96
+    assert form(t, M, K, N).startswith("fact_gemm ")
     rng = np.random.default_rng(200 + ex + 1000 * (200 + ew))
     x = rng.standard_normal((M, K)).astype(np.float32)
     v = rng.standard_normal((N, K)).astype(np.float32)
@@ -191,6 +206,7 @@ def test_fact_gemm_tiny_rows_large_scales(name):
     the outputs lie near 2^-90."""
     t = FACT[name]
     M, N, K = 40, 2500, 512
+    assert form(t, M, K, N).startswith("fact_gemm ")
     w = fact_weights(t, K, N, seed=7)
     _, size, at = BLOCK[t]
     for o in at:
@@ -213,6 +229,7 @@ def test_fact_gemm_all_rows_small(orc, name, M, N):
     scaled, and so is one infinite row's sign."""
     t = FACT[name]
     K = 512 if M > 16 else 1024
+    assert form(t, M, K, N).startswith("fact_gemm ")
     w = fact_weights(t, K, N, seed=2)
     x = np.random.default_rng(3).standard_normal((M, K)).astype(np.float32)
     y1 = gemm_dev(t, x, w, N)

@@ -3,7 +3,7 @@ small-M kernels) at the edges of its tiles and forms, against the oracle."""
 import numpy as np
 import pytest
 
-from hip_util import L, gemm_dev, normwise, quantize_dev, synth_weights, synth_x, to_dev
+from hip_util import form, gemm_dev, normwise, quantize_dev, synth_weights, synth_x
 from oracle.oracle import Q4_0, Q4_K, Q5_0, Q6_K, Q8_0
 
 pytestmark = pytest.mark.gpu
@@ -17,14 +17,27 @@ TOL = 4e-6
 
 # (M, N, K): one token and one row past a 32- and 64-tile, K ending inside a
 # 128-element stage (64-, 32- and 192-element tails), single-stage K, one stage
-# pair and its neighbours, M and N that take each form (32x32 with 8 and 4 K
-# groups, 64x64 with 2 and 1, 128x128)
+# pair and its neighbours, then M and N that take each form (32x32 with 8 and 4 K
+# groups, 64x64 with 2 and 1, 128x128: test_every_form_is_run)
 SHAPES32 = [(9, 31, 64), (12, 33, 192), (17, 1, 1088), (33, 65, 448), (65, 127, 2048), (5, 6555, 1088)]
 SHAPES256 = [(17, 33, 256), (33, 31, 512), (65, 129, 1280), (127, 64, 2048)]
-FORMS = [(31, 8200, 256), (40, 8200, 512), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256)]
-CASES = ([(t, *s) for t in (Q8_0, Q4_0) for s in SHAPES32] + [(Q5_0, M, N, K + 32 * (K < 2048)) for M, N, K in SHAPES32]
-         + [(Q6_K, *s) for s in SHAPES256] + [(t, *s) for t in NAMES if t != Q4_K for s in FORMS]
-         + [(Q4_K, *s) for s in ((65, 129, 1280), (127, 64, 2048), (33, 8200, 512), (96, 14400, 256), (130, 16300, 256))])
+FORMS = [(31, 8200, 256), (40, 8200, 512), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256), (500, 8190, 256)]
+TAILS = [(500, 8190, 192), (200, 24600, 320)]
+SHAPES = {t: SHAPES32 + FORMS + TAILS for t in (Q8_0, Q4_0)}
+SHAPES[Q5_0] = [(M, N, K + 32 * (K < 2048)) for M, N, K in SHAPES32 + TAILS] + FORMS
+SHAPES[Q6_K] = SHAPES256 + FORMS + [(70, 14400, 512)]
+SHAPES[Q4_K] = [(65, 129, 1280), (127, 64, 2048), (96, 4300, 512), (33, 8200, 512), (96, 14400, 256), (130, 16300, 256)]
+CASES = [(t, *s) for t in NAMES for s in SHAPES[t]]
+
+
+def test_every_form_is_run():
+    """The cases run each tile form of the product for each type (on 256 CUs)."""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the forms' lines depend on the CU count")
+    for t in NAMES:
+        got = {form(t, M, K, N) for M, N, K in SHAPES[t]}
+        assert got == {f"i8t {f}" for f in ("32x32x8", "32x32x4", "64x64x2", "64x64", "128x128")}, (NAMES[t], got)
 
 
 def weights(t, K, N, seed):
@@ -39,7 +52,7 @@ def weights(t, K, N, seed):
 def test_i8t_matches_oracle(orc, t, M, N, K):
     print(f"i8t {NAMES[t]} M={M} N={N} K={K}", flush=True)
     w = weights(t, K, N, seed=M + N + K + t)
-    assert L().lp_gemm_route(t, M, K, N, to_dev(w).data_ptr()).decode() == "i8mf"
+    assert form(t, M, K, N).startswith("i8t ")
     x = synth_x(M, K, seed=M + 1, outliers=0.01)
     x[M // 2, :32] = 0.0                                   # a block of zeros
     y = gemm_dev(t, x, w, N)
@@ -56,6 +69,7 @@ def test_i8t_rows_do_not_depend_on_their_neighbours(orc, t):
     K, N = 1024, 3000
     w = weights(t, K, N, seed=9 + t)
     x = synth_x(700, K, seed=10, outliers=0.01)
+    assert len({form(t, M, K, N) for M in (70, 129, 300, 700)}) >= 3
     first = gemm_dev(t, x[:70], w, N)
     for M in (129, 300, 700):
         y = gemm_dev(t, x[:M], w, N)
@@ -67,6 +81,7 @@ def test_i8t_non_finite_rows(orc, t):
     """A NaN or infinity in a row makes that row NaN as the reference's scale
     does, and leaves the others alone."""
     K, N, M = 512, 96, 70
+    assert form(t, M, K, N).startswith("i8t ")
     w = weights(t, K, N, seed=20 + t)
     x = synth_x(M, K, seed=21)
     x[3, 40] = np.nan
@@ -80,7 +95,7 @@ def test_i8t_non_finite_rows(orc, t):
 
 
 # each form, K ending inside a stage where the type allows it
-EDGE_SHAPES = [(9, 600, 192), (40, 8200, 192), (96, 4300, 320), (70, 14400, 192), (257, 16390, 192)]
+EDGE_SHAPES = [(9, 600, 192), (40, 8200, 192), (96, 4300, 320), (70, 14400, 192), (500, 8190, 192)]
 
 
 @pytest.mark.parametrize("wscale", [None, 2.0 ** -24, 6e4])
@@ -92,8 +107,7 @@ def test_i8t_tiny_rows(orc, t, M, N, K, wscale):
     print(f"i8t tiny rows {NAMES[t]} M={M} N={N} K={K}", flush=True)
     if t in (Q4_K, Q6_K):
         K, M = 512, max(M, 17 if t == Q6_K else 70)
-    if t == Q4_K and M > 200:                              # one round of 128 x 128 tiles
-        M, N = 130, 16300
+    assert form(t, M, K, N).startswith("i8t ")
     w = weights(t, K, N, seed=t).reshape(-1, {Q8_0: 34, Q4_0: 18, Q5_0: 22, Q4_K: 144, Q6_K: 210}[t])
     for at in {Q4_K: [0, 2], Q6_K: [208]}.get(t, [0]):
         if wscale:
@@ -160,8 +174,7 @@ def test_i8t_infinite_block_scales(t, M, N, K):
     print(f"i8t infinite scales {NAMES[t]} M={M} N={N} K={K}", flush=True)
     if t in (Q4_K, Q6_K):
         K, M = 512, max(M, 17 if t == Q6_K else 70)
-    if t == Q4_K and M > 200:
-        M, N = 130, 16300
+    assert form(t, M, K, N).startswith("i8t ")
     x = np.abs(synth_x(M, K, seed=31)) + 0.1
     x[2] = 0.0
     w, d = positive_weights(t, K, N, seed=t)

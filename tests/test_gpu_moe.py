@@ -155,7 +155,7 @@ def test_moe_empty():
 @pytest.mark.parametrize("multi", [False, True])
 def test_moe_many_pairs_per_expert_mfma(orc, multi):
     """When experts average more than 8 pairs (prefill-sized batches), Q4_K groups of
-    up to 16 pairs run on the small-M MFMA kernel: 8 experts, 96 tokens,
+    up to 32 pairs run on the tiled int8 product: 8 experts, 96 tokens,
     top-2, ragged groups, against the oracle."""
     t, E, T, topk, K, N = Q4_K, 8, 96, 2, 1024, 80
     w = synth_weights(t, K, N * E, seed=81 + multi)
@@ -168,12 +168,10 @@ def test_moe_many_pairs_per_expert_mfma(orc, multi):
 
 @pytest.mark.parametrize("K,N", [(256, 300), (768, 200), (2048, 96), (3072, 40)], ids=lambda v: str(v))
 def test_moe_mfma_row_sets(orc, K, N):
-    """The MFMA groups' workgroups take several row sets in turn, and at
-    short K split their waves into fewer K-slices and more row groups (K 256:
-    1 slice x 8 row groups, 768: 2 x 4, 2048: 8 x 1, 3072: 8 x 1 over 12
-    super-blocks): ragged N (a partial last row set, workgroups with fewer
-    sets), 6 experts, 64 tokens, top-2 (about 21 pairs per expert, so some
-    experts take two groups), against the oracle."""
+    """Groups of the tiled int8 product at short and long K (one stage pair, K 256,
+    to twelve) and ragged N (a tile of 128 weight rows cut off, and three of them):
+    6 experts, 64 tokens, top-2 (about 21 pairs per expert, so some experts take two
+    groups), against the oracle."""
     t, E, T, topk = Q4_K, 6, 64, 2
     w = synth_weights(t, K, N * E, seed=K + N)
     idx = routing(T, topk, E, seed=K)

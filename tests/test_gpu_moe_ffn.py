@@ -50,8 +50,8 @@ def run_both(orc, T, H, n_exp, top_k, inter, gu_t, dn_t, router_t, seed, paired_
     # Gemma4 26B layer shape (tests/bench_cpu_gpu.cpp:55-57): H 2816, 128
     # experts, top-8, expert inter 704 (down K = 704: a Q8_0 tensor)
     (2, 2816, 128, 8, 704, Q4_K, Q8_0, F32),
-    # 144 pairs over 16 experts (9 per expert): both expert passes on the MFMA
-    # group kernel
+    # 144 pairs over 16 experts (9 per expert): both expert passes on the tiled
+    # product, groups of 32
     (72, 512, 16, 2, 256, Q4_K, Q4_K, F32),
 ], ids=lambda v: str(v))
 def test_moe_ffn_matches_oracle(orc, T, H, n_exp, top_k, inter, gu_t, dn_t, router_t):
@@ -61,6 +61,30 @@ def test_moe_ffn_matches_oracle(orc, T, H, n_exp, top_k, inter, gu_t, dn_t, rout
     assert np.allclose(wts, rw, rtol=1e-5, atol=1e-7)
     assert np.isfinite(out).all()
     assert normwise(out, ref) <= 1e-4
+
+
+# passes of two types that want different groups: 5 pairs per expert 8 and 32 (both
+# take 4), 20 pairs 64 and 32, 100 pairs 128 and 64 or 64 and 128 (both take the
+# smaller), 128 twice; down K 704 ends inside a 128-element stage
+@pytest.mark.parametrize("T,inter,gu_t,dn_t,groups", [
+    (20, 704, Q4_K, Q8_0, (8, 32)), (20, 256, Q4_K, Q6_K, (8, 32)), (80, 256, Q8_0, Q4_K, (64, 32)),
+    (400, 704, Q4_K, Q8_0, (128, 64)), (400, 512, Q6_K, Q4_0, (128, 64)), (400, 256, Q8_0, Q6_K, (64, 128)),
+    (400, 256, Q4_K, Q6_K, (128, 128))], ids=lambda v: str(v))
+def test_moe_ffn_two_types(orc, T, inter, gu_t, dn_t, groups):
+    """Prompts whose expert passes take different group sizes, against the oracle. Most
+    tokens agree to fp32 rounding; where the two sides' GeGLU outputs lie on either side of
+    a rounding step of the int8 blocks, a code differs by one: one of inter inputs by a 127th
+    of its block's largest, about 3 / 127 of a typical one, i.e. 3 / (127 sqrt(inter)) of
+    the output, 1.5e-3 at inter 256."""
+    from hip_util import L
+    H, n_exp, top_k = 512, 8, 2
+    assert (L().lp_moe_group_pairs(gu_t, T, top_k, n_exp, H, 0), L().lp_moe_group_pairs(dn_t, T, top_k, n_exp, inter, 1)) == groups
+    (out, idx, wts), (ref, ridx, rw) = run_both(orc, T, H, n_exp, top_k, inter, gu_t, dn_t, F32, seed=T + inter + gu_t)
+    assert np.array_equal(idx, ridx)
+    assert np.allclose(wts, rw, rtol=1e-5, atol=1e-7)
+    err = np.abs(out - ref).max(1) / np.abs(ref).max(1)
+    print(f"token errors: median {np.median(err):.1e}, above 2e-5 {(err > 2e-5).mean():.3f}, largest {err.max():.1e}", flush=True)
+    assert np.median(err) <= 2e-5 and (err > 2e-5).mean() <= 0.05 and err.max() <= 3 * 3 / (127 * inter ** 0.5)
 
 
 @pytest.mark.parametrize("T,top_k", [(1, 3), (3, 5), (9, 3)])

@@ -35,8 +35,19 @@ def pairs_of(counts, topk, rng):
 
 
 # pairs per expert: means that take groups of 32, 64 and 128 (8 experts), with empty
-# experts, one pair, whole groups and one pair past them
+# experts, one pair, whole groups and one pair past them. Q8_0 and Q4_0 go over to 64 at
+# 16 pairs per expert and stay there.
 COUNTS = {32: [0, 1, 32, 33, 64, 5, 31, 18], 64: [0, 1, 64, 65, 128, 30, 63, 97], 128: [0, 1, 128, 129, 257, 60, 255, 130]}
+SMALL = {**COUNTS, 32: [0, 1, 32, 33, 10, 5, 20, 18]}
+
+
+def counts_of(t, gs):
+    return (SMALL if t in (Q8_0, Q4_0) else COUNTS)[gs]
+
+
+def check_group(t, idx, E, K, multi, gs):
+    want = 64 if t in (Q8_0, Q4_0) and gs == 128 else gs
+    assert L().lp_moe_group_pairs(t, *idx.shape, E, K, multi) == want
 
 
 @pytest.mark.parametrize("multi", [0, 1])
@@ -49,8 +60,9 @@ def test_moe_tile_matches_oracle(orc, t, multi, gs, topk, K, N):
         K += 64                                    # K ends inside a 128-element stage
     rng = np.random.default_rng(gs + K + N + t)
     E = 8
-    idx = pairs_of(COUNTS[gs], topk, rng)
+    idx = pairs_of(counts_of(t, gs), topk, rng)
     T = idx.shape[0]
+    check_group(t, idx, E, K, multi, gs)
     w = synth_weights(t, K, E * N, seed=t + gs)
     x = synth_x(T * topk if multi else T, K, seed=5, outliers=0.01)
     y = grouped(t, x, multi, idx, w, E, K, N)
@@ -89,7 +101,8 @@ def test_moe_tile_infinite_block_scales(t, gs, multi):
     a NaN activation row is NaN."""
     rng = np.random.default_rng(gs)
     E, K, N, topk = 8, 512, 70, 2
-    idx = pairs_of(COUNTS[gs], topk, rng)
+    idx = pairs_of(counts_of(t, gs), topk, rng)
+    check_group(t, idx, E, K, multi, gs)
     P = idx.size
     x = np.abs(synth_x(P if multi else len(idx), K, seed=6)) + 0.1
     w, d = positive_weights(t, K, E * N, seed=gs)
