@@ -775,6 +775,8 @@ bool fact_gemm_preferred(uint32_t type, int M, int K, int N) {
     const long cus = device_cu_count(), rounds = ((long)((M + 31) / 32) * ((N + 31) / 32) + cus - 1) / cus;
     const bool many = type == T_F32 || type == T_F16;
     const long line = many ? 12000 + 37000 * rounds : type == T_Q2_K ? 32000 : 24000;
+    // a tile's weight rows (128) and x rows (128) are addressed with 32-bit offsets
+    if (128 * fact_row_bytes(type, K) > (1ull << 32) || K > 1 << 25) return false;
     return M >= (type == T_F16 ? 6 : 5) && (long)M * N >= (K <= 2048 ? 2 * line : line);
 }
 
