@@ -695,7 +695,7 @@ const char* lp_gemm_form(uint32_t type, int M, int K, int N, const void* w) {
     const uint8_t* wb = static_cast<const uint8_t*>(w);
     if (check_shape(type, wb, M, K, N) != LP_OK || M <= 0 || N <= 0) return "";
     if (fact_type(type)) return fact_gemm_preferred(type, M, K, N) ? fact_gemm_form(type, M, N) : "fact";
-    if (use_i8t(type, M, K, N)) return i8t_form(type, M, N);
+    if (use_i8t(type, M, K, N)) return i8t_form(type, M, K, N);
     return gemm_q_route(type, M, K, N, wb);
 }
 

@@ -738,14 +738,21 @@ namespace {
 //   Q8_0 N 4096 M 512    (t64 512)   64x64 46.2  64x64x2 52.7  128x128 69
 //   Q8_0 N 4096 M 1024   (t128 256)  128x128 76.9  64x64 83.9
 //   Q6_K N 14336 M 2048  (t128 1792) 128x128 740  64x64 830
-enum Form { F32X32X8, F32X32X4, F64X64X2, F64X64, F128X128 };
+// Short rows have fewer stage pairs than eight groups: with four the call loses the
+// idle ones and half the last sum (kernel time with the quantizer, M 12, N 2048: K 256
+// 8.3 -> 7.1, K 1024 8.6 -> 7.3, Q6_K 10.3 -> 8.4; K 1536 8.6 against 9.0), and where one
+// pair is all of K and there are more tiles than CUs, four waves side by side read x once
+// (Q6_K N 14336 K 256 10.2 -> 8.8, N 32768 16.3 -> 9.1, Q4_0 12.6 -> 7.5; at K 512 only
+// from four tiles per CU, Q6_K N 32768 16.0 -> 11.9, N 14336 slower).
+enum Form { F32X128, F32X32X8, F32X32X4, F64X64X2, F64X64, F128X128 };
 
-Form pick_form(uint32_t type, int M, int N) {
+Form pick_form(uint32_t type, int M, int K, int N) {
     const long cus = device_cu_count();
     auto tiles = [&](int b) { return (long)((M + b - 1) / b) * ((N + b - 1) / b); };
     // one 32 x 32 tile per CU: eight waves share its K; two per CU (or at most
     // 32 rows, where larger tiles are half padding): four waves
-    if (tiles(32) <= cus) return F32X32X8;
+    if (tiles(32) <= cus) return K <= 1024 ? F32X32X4 : F32X32X8;
+    if (M <= 32 && (K <= 256 || (K <= 512 && tiles(32) >= 4 * cus))) return F32X128;
     if (tiles(32) <= 2 * cus || M <= 32) return F32X32X4;
     if (tiles(64) <= cus) return F64X64X2;
     // two 64 x 64 workgroups per CU against one of 128 x 128, which does four
@@ -761,6 +768,8 @@ Form pick_form(uint32_t type, int M, int N) {
 template <uint32_t T>
 hipError_t launch_t(const I8tArgs& g, Form f, hipStream_t st) {
     switch (f) {
+        // (Q4_K comes here with more than 32 rows)
+        case F32X128: if constexpr (T != T_Q4_K) return launch_cfg<T, 1, 1, 1, 4, 1>(g, st); return hipErrorInvalidValue;
         case F32X32X8: return launch_cfg<T, 1, 1, 1, 1, 8>(g, st);
         case F32X32X4: return launch_cfg<T, 1, 1, 1, 1, 4>(g, st);
         case F64X64X2: return launch_cfg<T, 1, 1, 2, 2, 2>(g, st);
@@ -804,8 +813,9 @@ bool i8t_preferred(uint32_t type, int M, int K, int N) {
     return false;
 }
 
-const char* i8t_form(uint32_t type, int M, int N) {
-    switch (pick_form(type, M, N)) {
+const char* i8t_form(uint32_t type, int M, int K, int N) {
+    switch (pick_form(type, M, K, N)) {
+        case F32X128: return "i8t 32x128";
         case F32X32X8: return "i8t 32x32x8";
         case F32X32X4: return "i8t 32x32x4";
         case F64X64X2: return "i8t 64x64x2";
@@ -818,7 +828,7 @@ hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, fl
                            hipStream_t st) {
     if (M <= 0 || N <= 0) return hipSuccess;
     I8tArgs g{w, A, y, M, N, K, row_bytes(type, K)};
-    const Form f = pick_form(type, M, N);
+    const Form f = pick_form(type, M, K, N);
     switch (type) {
         case T_Q8_0: return launch_t<T_Q8_0>(g, f, st);
         case T_Q4_0: return launch_t<T_Q4_0>(g, f, st);

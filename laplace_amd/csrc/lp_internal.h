@@ -103,7 +103,7 @@ bool i8mf_supported(uint32_t type, int M, int K, int N, const uint8_t* w);
 // Tiled int8 MFMA product of the quantized blocks (lp_gemm_i8t.hip) for all five
 // int8 types; i8t_preferred: the shapes where it is the fastest kernel.
 bool i8t_preferred(uint32_t type, int M, int K, int N);
-const char* i8t_form(uint32_t type, int M, int N);            // its tile form (lp_gemm_form)
+const char* i8t_form(uint32_t type, int M, int K, int N);     // its tile form (lp_gemm_form)
 hipError_t launch_gemm_i8t(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,
                            hipStream_t st);
 hipError_t launch_gemv_i8mf(uint32_t type, const uint8_t* w, const ActView& A, float* y, int M, int K, int N,

@@ -4,7 +4,7 @@ import pytest
 
 from laplace_amd import _lib
 
-F32, F16, BF16, Q2_K, Q5_K = 0, 1, 30, 10, 13
+F32, F16, Q4_0, Q8_0, Q2_K, Q5_K, Q6_K, BF16 = 0, 1, 2, 8, 10, 13, 14, 30
 
 
 # the longest rows whose 128-row tile offsets stay within 32 bits: 2^25 bytes of weights,
@@ -14,3 +14,16 @@ def test_fact_gemm_row_offsets_fit_32_bits(t, longest):
     L = _lib.lib()
     assert L.lp_gemm_form(t, 2048, longest, 2048, None).startswith(b"fact_gemm ")
     assert L.lp_gemm_form(t, 2048, longest + 256, 2048, None) == b"fact"
+
+
+# (type, M, K, N) on a 256-CU part, in pairs on either side of a line
+@pytest.mark.parametrize("call,form", [
+    ((Q8_0, 12, 1024, 2048), "i8t 32x32x4"), ((Q8_0, 12, 1088, 2048), "i8t 32x32x8"),
+    ((Q6_K, 16, 1024, 4096), "i8t 32x32x4"), ((Q6_K, 17, 1280, 4096), "i8t 32x32x8"),
+    ((Q6_K, 9, 256, 14336), "i8t 32x128"), ((Q6_K, 9, 512, 14336), "i8t 32x32x4"),
+    ((Q4_0, 5, 512, 32768), "i8t 32x128"), ((Q4_0, 5, 576, 32768), "i8t 32x32x4"),
+])
+def test_short_rows_take_fewer_k_groups(call, form):
+    """Where a row has too few stages for eight groups of waves to share."""
+    t, M, K, N = call
+    assert _lib.lib().lp_gemm_form(t, M, K, N, None).decode() == form

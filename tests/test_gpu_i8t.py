@@ -17,8 +17,8 @@ TOL = 4e-6
 
 # (M, N, K): one token and one row past a 32- and 64-tile, K ending inside a
 # 128-element stage (64-, 32- and 192-element tails), single-stage K, one stage
-# pair and its neighbours, then M and N that take each form (32x32 with 8 and 4 K
-# groups, 64x64 with 2 and 1, 128x128: test_every_form_is_run)
+# pair and its neighbours, then M and N that take each form (32x128, 32x32 with 8 and
+# 4 K groups, 64x64 with 2 and 1, 128x128: test_every_form_is_run)
 SHAPES32 = [(9, 31, 64), (12, 33, 192), (17, 1, 1088), (33, 65, 448), (65, 127, 2048), (5, 6555, 1088)]
 SHAPES256 = [(17, 33, 256), (33, 31, 512), (65, 129, 1280), (127, 64, 2048)]
 FORMS = [(31, 8200, 256), (40, 8200, 512), (33, 14400, 256), (96, 16500, 256), (200, 24600, 256), (500, 8190, 256)]
@@ -37,7 +37,8 @@ def test_every_form_is_run():
         pytest.skip("the forms' lines depend on the CU count")
     for t in NAMES:
         got = {form(t, M, K, N) for M, N, K in SHAPES[t]}
-        assert got == {f"i8t {f}" for f in ("32x32x8", "32x32x4", "64x64x2", "64x64", "128x128")}, (NAMES[t], got)
+        want = {f"i8t {f}" for f in ("32x128", "32x32x8", "32x32x4", "64x64x2", "64x64", "128x128")}
+        assert got == want - ({"i8t 32x128"} if t == Q4_K else set()), (NAMES[t], got)
 
 
 def weights(t, K, N, seed):
@@ -95,7 +96,7 @@ def test_i8t_non_finite_rows(orc, t):
 
 
 # each form, K ending inside a stage where the type allows it
-EDGE_SHAPES = [(9, 600, 192), (40, 8200, 192), (96, 4300, 320), (70, 14400, 192), (500, 8190, 192)]
+EDGE_SHAPES = [(9, 600, 1216), (17, 33000, 192), (40, 8200, 192), (96, 4300, 320), (70, 14400, 192), (500, 8190, 192)]
 
 
 @pytest.mark.parametrize("wscale", [None, 2.0 ** -24, 6e4])
@@ -105,8 +106,10 @@ def test_i8t_tiny_rows(orc, t, M, N, K, wscale):
     """Rows down to the smallest fp32 values keep their products' 24 bits, whatever the
     block scales of the weights; the rows beside them keep their bits."""
     print(f"i8t tiny rows {NAMES[t]} M={M} N={N} K={K}", flush=True)
+    if t == Q4_K and N == 33000:
+        pytest.skip("Q4_K has no 32 x 128 tiles")
     if t in (Q4_K, Q6_K):
-        K, M = 512, max(M, 17 if t == Q6_K else 70)
+        K, M = 1280 if K > 512 else 512, max(M, 17 if t == Q6_K else 70)
     assert form(t, M, K, N).startswith("i8t ")
     w = weights(t, K, N, seed=t).reshape(-1, {Q8_0: 34, Q4_0: 18, Q5_0: 22, Q4_K: 144, Q6_K: 210}[t])
     for at in {Q4_K: [0, 2], Q6_K: [208]}.get(t, [0]):
@@ -172,8 +175,10 @@ def test_i8t_infinite_block_scales(t, M, N, K):
     (whose kernels multiply a row's last block with zeros once more past its end, which is
     left out here); the other weight rows keep their bits."""
     print(f"i8t infinite scales {NAMES[t]} M={M} N={N} K={K}", flush=True)
+    if t == Q4_K and N == 33000:
+        pytest.skip("Q4_K has no 32 x 128 tiles")
     if t in (Q4_K, Q6_K):
-        K, M = 512, max(M, 17 if t == Q6_K else 70)
+        K, M = 1280 if K > 512 else 512, max(M, 17 if t == Q6_K else 70)
     assert form(t, M, K, N).startswith("i8t ")
     x = np.abs(synth_x(M, K, seed=31)) + 0.1
     x[2] = 0.0
