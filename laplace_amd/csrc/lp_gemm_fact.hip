@@ -761,23 +761,42 @@ hipError_t launch_t(const FactArgs& g, hipStream_t st) {
 }  // namespace
 
 // Where this product beats the GEMVs, which read the weights once per 4 rows: up to
-// 32 rows its time depends on K alone (one round of tiles), theirs on M N K, so the
-// line is a number of outputs, for F16 and F32 one per round of tiles; twice as many at K <= 2048, where its launch and last
-// reduction weigh more. Measured (us, GEMV against this): K 4096: BF16 N 4096 M 5
-// 18.7 / 19, M 6 21.0 / 19.5, M 12 31.5 / 18.8, M 33 82.5 / 20.0; N 1024 M 12 9.2 /
-// 19, M 33 23.4 / 18.3; Q5_K N 4096 M 6 30.4 / 27.7, M 12 66 / 28; Q3_K M 6 29.1 /
-// 26.9; Q2_K M 6 22.3 / 26, M 8 28.9 / 26.9; F16, F32 (more products) N 4096 M 8
-// 24.4, 28.7 / 32, 37, M 12 37.4, 40.5 / 32.1, 36.5; N 14336 (two rounds of tiles) F16
-// M 6 65.8 / 62.8, F32 M 6 86 / 73, N 8200 F16 M 8 52.5 / 61. K 1024, N 4096: BF16 M 8 7.9 / 7.2, M 12 10.5 / 7.2; F16 M 12 11.2 / 11.5,
-// M 33 27 / 11.5. Large: N 14336 K 4096 M 200 BF16 1690 -> 140, Q5_K 2660 -> 186, Q3_K
-// 2018 -> 150, Q2_K 1556 -> 168, F16 1547 -> 280, F32 2057 -> 329.
+// 32 rows its time depends on K alone and on the rounds of tiles, theirs on M N K, so the
+// line is a number of outputs (for F16, F32, Q2_K and Q5_K one per round of tiles), twice as
+// many at K <= 2048, where its launch and last reduction weigh more. Measured (us, GEMV
+// against this):
+//   BF16 K 4096: N 4096 M 5 18.7 / 19, M 6 21.0 / 19.5, M 12 31.5 / 18.8, M 33 82.5 / 20.0; N 1024
+//     M 12 9.2 / 19, M 33 23.4 / 18.3. Whole passes of 4 rows cost the GEMV less: N 2048 M 12 15.5 /
+//     18.5, M 13 19.4 / 18.6, M 16 19.6 / 18.7; N 3072 M 8 15.7 / 18.7, M 9 19.9 / 18.8; not at K 8192,
+//     N 3072 M 8 36.0 / 32.9.
+//   Q5_K K 4096: N 4096 M 6 30.4 / 27.7, M 12 66 / 28; K 3072: N 3072 M 8 20.6 / 22.0, M 9 25.2 / 22.3,
+//     two rounds N 10240 M 6 38.3 / 39.6, M 7 41.1 / 39.5; K 2048 N 10240 M 8 22.6 / 27.9, M 9 29.1 /
+//     28.0, N 14336 M 6 26.2 / 28.3, M 7 28.7 / 28.1; K 1024 N 10240 M 5 17.7 / 16.0.
+//   Q2_K K 4096: N 4096 M 6 22.3 / 26, M 8 28.9 / 26.9, two rounds N 10240 M 6 40.3 / 48.9, M 7 51.8 /
+//     48.8; K 2048 N 10240 M 8 22.9 / 26.7, M 9 29.0 / 26.7, N 14336 M 6 25.6 / 26.7, M 7 28.3 / 26.6.
+//   Q3_K K 4096 N 4096 M 6 29.1 / 26.9.
+//   F16, F32 (more products) K 4096: N 4096 M 8 24.4, 28.7 / 32, 37, M 12 37.4, 40.5 / 32.1, 36.5; F16
+//     N 3072 M 16 29.5 / 31.5, K 8192 73.7 / 61.2; N 14336 (two rounds of tiles) F16 M 6 65.8 / 62.8, F32 M 6 86 / 73,
+//     N 8200 F16 M 8 52.5 / 61.
+//   K 1024, N 4096: BF16 M 8 7.9 / 7.2, M 12 10.5 / 7.2; F16 M 12 11.2 / 11.5, M 33 27 / 11.5.
+// Large: N 14336 K 4096 M 200 BF16 1690 -> 140, Q5_K 2660 -> 186, Q3_K 2018 -> 150, Q2_K
+// 1556 -> 168, F16 1547 -> 280, F32 2057 -> 329.
 bool fact_gemm_preferred(uint32_t type, int M, int K, int N) {
     const long cus = device_cu_count(), rounds = ((long)((M + 31) / 32) * ((N + 31) / 32) + cus - 1) / cus;
-    const bool many = type == T_F32 || type == T_F16;
-    const long line = many ? 12000 + 37000 * rounds : type == T_Q2_K ? 32000 : 24000;
     // a tile's weight rows (128) and x rows (128) are addressed with 32-bit offsets
     if (128 * fact_row_bytes(type, K) > (1ull << 32) || K > 1 << 25) return false;
-    return M >= (type == T_F16 ? 6 : 5) && (long)M * N >= (K <= 2048 ? 2 * line : line);
+    const long many = 12000 + 37000 * rounds;
+    long line = 24000;
+    switch (type) {
+        case T_F32: line = many; break;
+        case T_F16: line = N < 4096 && K > 2048 && K < 6144 && many < 50000 ? 50000 : many; break;
+        case T_BF16: if (K > 2048 && K <= 6144 && M % 4 == 0) line = 30000; break;
+        case T_Q2_K: line = K > 2048 ? 32000 * rounds : 32000; break;
+        case T_Q5_K: if (K > 2048 && K < 4096) line = rounds > 1 ? 31000 * rounds : 25000; break;
+    }
+    if (K <= 2048) line *= 2;
+    if ((type == T_Q2_K || type == T_Q5_K) && K > 1024 && K <= 2048 && rounds > 1) line = 45000 * rounds;
+    return M >= (type == T_F16 ? 6 : 5) && (long)M * N >= line;
 }
 
 const char* fact_gemm_form(uint32_t type, int M, int N) {

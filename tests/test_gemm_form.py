@@ -27,3 +27,16 @@ def test_short_rows_take_fewer_k_groups(call, form):
     """Where a row has too few stages for eight groups of waves to share."""
     t, M, K, N = call
     assert _lib.lib().lp_gemm_form(t, M, K, N, None).decode() == form
+
+
+@pytest.mark.parametrize("t,M,K,N,tiled", [
+    (BF16, 12, 4096, 2048, False), (BF16, 13, 4096, 2048, True), (BF16, 16, 4096, 2048, True), (BF16, 8, 3072, 3072, False),
+    (BF16, 6, 4096, 4096, True), (BF16, 8, 4096, 4096, True),
+    (Q5_K, 8, 3072, 3072, False), (Q5_K, 9, 3072, 3072, True), (Q5_K, 6, 3072, 10240, False), (Q5_K, 7, 3072, 10240, True),
+    (Q5_K, 8, 2048, 10240, False), (Q5_K, 9, 2048, 10240, True), (Q5_K, 5, 1024, 10240, True), (Q5_K, 6, 4096, 4096, True),
+    (Q2_K, 6, 4096, 10240, False), (Q2_K, 7, 4096, 10240, True), (Q2_K, 6, 2048, 14336, False), (Q2_K, 7, 2048, 14336, True),
+    (F16, 16, 4096, 3072, False), (F16, 12, 4096, 4096, True), (F16, 16, 8192, 3072, True), (BF16, 8, 8192, 3072, True)])
+def test_fact_gemm_lines(t, M, K, N, tiled):
+    """The tiled product takes calls where it measured faster than the GEMVs."""
+    got = _lib.lib().lp_gemm_form(t, M, K, N, None).decode()
+    assert got.startswith("fact_gemm ") if tiled else got == "fact"
