@@ -797,16 +797,33 @@ hipError_t launch_t(const I8tArgs& g, Form f, hipStream_t st) {
 // and for K > 4096 not where that round would be half empty (N 14336 M 64 42 -> 27,
 // M 256 82 -> 74.5, M 512 108 against 143 here; N 4096 M 512 59 -> 48, M 1024 94
 // -> 77; N 4096 K 14336 M 256 102 -> 87, M 512 146 against 154 here, M 1024 266
-// -> 250): beyond, the split-precision kernels' cheaper epilogue wins.
+// -> 250): beyond, the split-precision kernels' cheaper epilogue wins. It also wins at
+// long K where this product's tiles are mostly padding: up to 64 rows on more than a 64 x 64
+// tile per CU (K 4096: N 18944 M 33 39 / 48, M 64 46 / 48, N 28672 M 33 43 / 48, M 56 48 / 49, N 32768
+// M 40 50 / 49; K 3072: N 24576 M 40 35 / 38, N 28672 M 48 39 / 39, N 32768 M 33 40 / 39; K 2048:
+// N 18944 M 33 25 / 26, M 64 32 / 27), and 129..192 rows where the wide-token kernel fills the
+// CUs (K 4096: N 14336 M 129 63 / 72, M 176 69 / 72, M 192 72 / 73, N 16384 M 144 70 / 72, M 160 74 / 72,
+// N 12288, not that kernel, 81 / 72; K 5120 N 14336 M 129 78 / 88; K 3072 N 14336 M 129 53 / 56, M 160
+// 57 / 56; K 2048 43 / 39).
+// Q4_0 rows beyond 12000 on few weight rows: the GEMVs' two passes do not grow with K there
+// (N 512 K 14336 M 9 18.5 / 22.3, M 12 21.7 / 22.5, M 13 22.8 / 22.5; K 18944 M 12 22.0 / 29.2; N 768
+// K 14336 M 11 20.8 / 22.5, K 18944 M 9 30.7 / 29.1; N 1024 K 14336 M 9 22.3 / 22.5, M 10 25.1 / 22.5).
 bool i8t_preferred(uint32_t type, int M, int K, int N) {
     const long cus = device_cu_count();
     switch (type) {
-        case T_Q8_0: case T_Q4_0: case T_Q5_0:
+        case T_Q4_0:
+            if (M <= 16 && N <= (K <= 16384 ? 768 : 512) && K > 650 * (10 + M)) return false;
+            [[fallthrough]];
+        case T_Q8_0: case T_Q5_0:
             return M > 8 || (M >= 5 && (long)M * N >= (type == T_Q5_0 || K < 2048 ? 32768 : 20000));
         case T_Q6_K: return M > 16 || (M >= (K < 2048 ? 16 : 13) && K >= 1024) || (M >= 9 && (N + 31) / 32 > cus);
         case T_Q4_K: {
             if (M <= 32 || (M <= 64 && N <= 4096)) return false;
             const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+            const long mn = (long)M * N;
+            if (K >= 3072 && M <= 64 && t64 > cus && mn <= (K >= 4096 ? 1500000 : 1200000)) return false;
+            if (K >= 3072 && M > 128 && M <= 192 && wt_auto_cfg(M, K, N) == 0 && mn <= (K >= 4096 ? 2600000 : 2100000))
+                return false;
             return t128 <= cus && (K <= 4096 || t64 <= cus || 4 * t128 > 3 * cus);
         }
     }

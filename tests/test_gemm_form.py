@@ -4,7 +4,7 @@ import pytest
 
 from laplace_amd import _lib
 
-F32, F16, Q4_0, Q8_0, Q2_K, Q5_K, Q6_K, BF16 = 0, 1, 2, 8, 10, 13, 14, 30
+F32, F16, Q4_0, Q8_0, Q2_K, Q4_K, Q5_K, Q6_K, BF16 = 0, 1, 2, 8, 10, 12, 13, 14, 30
 
 
 # the longest rows whose 128-row tile offsets stay within 32 bits: 2^25 bytes of weights,
@@ -40,3 +40,14 @@ def test_fact_gemm_lines(t, M, K, N, tiled):
     """The tiled product takes calls where it measured faster than the GEMVs."""
     got = _lib.lib().lp_gemm_form(t, M, K, N, None).decode()
     assert got.startswith("fact_gemm ") if tiled else got == "fact"
+
+
+@pytest.mark.parametrize("t,M,K,N,tiled", [
+    (Q4_K, 33, 4096, 18944, False), (Q4_K, 48, 4096, 32768, True), (Q4_K, 33, 2048, 18944, True), (Q4_K, 33, 4096, 14336, True),
+    (Q4_K, 130, 4096, 14336, False), (Q4_K, 192, 4096, 14336, True), (Q4_K, 130, 4096, 12288, True), (Q4_K, 130, 2048, 14336, True),
+    (Q4_K, 128, 4096, 14336, True), (Q4_K, 160, 3072, 14336, True), (Q4_K, 130, 3072, 14336, False),
+    (Q4_0, 9, 14336, 512, False), (Q4_0, 13, 14336, 512, True), (Q4_0, 12, 18944, 512, False), (Q4_0, 9, 18944, 768, True),
+    (Q4_0, 9, 10240, 512, True), (Q4_0, 17, 18944, 512, True)])
+def test_int8_product_lines(t, M, K, N, tiled):
+    """The tiled int8 product takes calls where it measured faster than the kernels beside it."""
+    assert _lib.lib().lp_gemm_form(t, M, K, N, None).decode().startswith("i8t ") == tiled
