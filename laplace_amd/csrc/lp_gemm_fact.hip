@@ -21,11 +21,11 @@
 // LDS in operand order ([32 rows][16 k][half][row][8 bf16]); the next stage is in
 // registers meanwhile.
 //
-// What bounds it (BF16, N 4096 K 4096 M 512, 95 us of which ~7 launch: 540 TFLOP/s of
-// bf16 products, the GEMVs 1205 us, one pass over the weights per 4 rows): loads are
+// What bounds it (BF16, N 4096 K 4096 M 512, 87 us, 590 TFLOP/s of bf16 products, the
+// GEMVs 1175 us, one pass over the weights per 4 rows; matrix unit busy 21 %): loads are
 // hidden behind the products; splitting x and writing its planes (58 us alone) and the
 // products (72 - 80 us alone) follow each other in every wave. Large: M 2048 N 14336
-// 15890 -> 928 us, Q5_K N 4096 K 14336 M 2048 95144 -> 1253. Normwise errors against
+// 15890 -> 884 us, Q5_K N 4096 K 14336 M 2048 95144 -> 1230. Normwise errors against
 // 64-bit sums 5e-8 .. 1e-7, the GEMVs' 0.7e-7 .. 3e-7.
 #include <hip/hip_runtime.h>
 
@@ -716,7 +716,7 @@ namespace {
 //   BF16  M 64   (256 tiles of 32 x 32)   32x32x8 24.8, 32x32x4 30, 64x64x2 49
 //         M 128  (512)                    32x32x4 41, 32x32x8 47, 64x64x2 51
 //         M 256  (256 tiles of 64 x 64)   64x64x2 54, 64x64 76, 32x32x4 77
-//         M 512  (512)                    64x64 95, 64x64x2 107, 128x128 123
+//         M 512  (512)                    64x64 95 (87 in a stream of calls), 64x64x2 107, 128x128 123
 //         M 2048 (512 tiles of 128 x 128) 128x128 253, 64x64 343
 //   F32   M 128  32x32x6 85, 64x64 119      M 256  64x64 119, 64x128 165
 //         M 512  64x128 169, 64x64 225

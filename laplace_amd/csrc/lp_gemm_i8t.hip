@@ -26,8 +26,8 @@
 // VALU forms that run at twice the rate of the three-operand ones (2.4 - 2.9
 // against 4.3 cycles per wave measured).
 //
-// What bounds it (Q8_0, N 14336 K 4096 M 2048: 460 us, 520 TOPS; the chunked
-// kernels it replaces 4170 us, which streamed the weights 64 times): with the
+// What bounds it (Q8_0, N 14336 K 4096 M 2048: 505 us a call with the quantizer, 480
+// TOPS; the chunked kernels it replaces 4170 us, which streamed the weights 64 times): with the
 // products removed the loads and LDS writes alone take 350 of 128 x 128 tiles'
 // time, with the loads removed the products 290; of the loads the 34-byte weight
 // blocks are two thirds (64 rows touch 64 cache lines per load), so weights are
@@ -789,9 +789,9 @@ hipError_t launch_t(const I8tArgs& g, Form f, hipStream_t st) {
 // Q5_0 69 -> 18.9; Q8_0's 16-row kernel 54.9 -> 17.0; N 1024 K 1024 8.5 -> 8.3).
 // Q6_K from 9 rows where 32-row tiles fill the CUs (N 14336 M 9 37.0 -> 20.6), else
 // from 13 (K 4096, N 512 .. 4096: M 13 13.8 -> 13.2, M 17 18.8 -> 13.3, N 4096 M 512
-// 382 -> 65; N 3584 K 18944 M 512 1327 -> 270). Short rows (K 1024: M 16 8.5 against
-// 9.8 here, M 17 12.8 -> 9.9) stay there up to 15 rows, and 16 below K = 1024: from
-// there on, 16 rows give the bits of the first 16 of a longer prompt.
+// 382 -> 65; N 3584 K 18944 M 512 1327 -> 270). Short rows (K 1024: M 13 8.6 / 8.7,
+// M 16 8.8 / 8.4; K 1536 M 16 9.3 / 10.5) stay there up to 15 rows, and 16 below K = 1024:
+// from there on, 16 rows give the bits of the first 16 of a longer prompt.
 // Q4_K where the 16-row chunks of the small-M kernel end (beyond 32 rows, 64 for
 // up to 4096 weight rows) while one round of 128 x 128 tiles covers the product,
 // and for K > 4096 not where that round would be half empty (N 14336 M 64 42 -> 27,
