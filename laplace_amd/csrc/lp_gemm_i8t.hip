@@ -317,6 +317,8 @@ __device__ __forceinline__ void w_store(const WReg<T>& r, uint8_t* st, int n, in
 // block scale has no pieces (inf - inf), so its product above is NaN where the plain
 // one is an infinity: non-finite outputs are made again here, except in rows whose
 // own scales are not finite (a NaN or infinite activation), which are NaN either way.
+// Measured (us a call, Q8_0 N 4096 K 4096 M 512, plain 45 - 50): one infinite scale in the
+// matrix 89, a NaN activation row 48; N 14336 M 2048 504, 516 with one infinite scale.
 template <uint32_t T>
 __device__ __forceinline__ float wave_dot(const ActView& A, int arow, const uint8_t* wrow, int K, int lane) {
     float s = 0.0f;
